@@ -64,7 +64,23 @@ struct BinGeom {
   int sp_pp;
   int sp_gc;
   unsigned char sp_lane[192];
+  // 1: matrix-core B and B^T (mx.hpp), d = 3.  Bins are then ragged along
+  // dimensions 1 and 2 (bin b of nb_t holds cells mx_lo(b) .. mx_lo(b+1)-1,
+  // bs_t of them at most), numbered with dimension 0 fastest, so that a
+  // column's nodes are contiguous and sorted by their dimension-0 cell.
+  // mx_span: bins per dimension whose tiles may reach a bin's cells (all of
+  // them where that is fewer).
+  int mx;
+  int mx_span[3];
 };
+
+// Ragged bins: first cell of bin b of nb over n cells, and the bin of cell c
+// (n <= kMxMaxN, so that the products fit an int)
+constexpr int kMxMaxN = 32767;
+__host__ __device__ inline int mx_lo(int b, int n, int nb) { return b * n / nb; }
+__host__ __device__ inline int mx_bin(int c, int n, int nb) { return ((c + 1) * nb - 1) / n; }
+// widest window of the matrix-core kernels: m = kMxMaxM
+constexpr int kMxMaxM = 6;
 
 // Kaiser-Bessel window of one dimension, scaled by 1/phi(0) so that the B
 // weights stay O(1) (the scale is folded into the deconvolution factors).
@@ -213,6 +229,26 @@ template <typename R> struct Engine {
   cplx<R> *tiles = nullptr;
   long tiles_cap = 0;
   bool tile_scratch = false;
+  // complex values of the scratch tiles of one right-hand side
+  long tile_cells = 0;
+  // matrix-core path: per spreading item (in bin order) its first plane in
+  // the scratch tiles, its first node's dimension-0 cell, its plane count
+  int4 *mx_info = nullptr;
+  long mx_info_cap = 0;
+  // the same per spreading bin (z = 0: no nodes): its item's, or for a bin of
+  // several items those of the tile their planes are summed into; the bins of
+  // several items
+  bool mx_dense = false;  // several nodes per occupied cell: see bin_nodes
+  int4 *mx_bin_info = nullptr;
+  int *mx_multi = nullptr;
+  long mx_bins_cap = 0, mx_multi_n = 0;
+  // the bins that the LDS-tile kernels would use for a matrix-core plan, and
+  // whether they would run its batches in one launch: the allocation-free
+  // batched adjoint accepts the same plans whichever kernels run
+  BinGeom tile_geom{};
+  bool tile_batchable = false;
+  int tile_spread_max_per_sub = 0;
+  long tile_items = 0;  // spreading items in those bins
   int *scratch_i = nullptr;  // binning scratch
   int *zone_tab = nullptr;   // geom.zmap and geom.zdesc
   int2 *slots = nullptr, *islots = nullptr;  // geom.slots, geom.islots
@@ -265,6 +301,7 @@ template <typename R> struct Engine {
 
   void create(int d_, const long *N_, const long *n_, long M_, int m_);
   void set_bins(const int *bs);
+  void set_mx_bins();
   void destroy();
   void upload_nodes(const R *x_host);
   void build_nodes();  // from xdev
@@ -295,6 +332,7 @@ template <typename R> struct Engine {
   int device = 0;
   void *noalloc_scratch = nullptr;  // device address of the scratch array
   long noalloc_bytes_per_rhs() const;
+  long noalloc_limit_bytes() const;
   int adjoint_batch_noalloc(const cplx<R> *f_dev, cplx<R> *fhat_dev, int nrhs);
   cplx<R> *bgrid = nullptr;   // batched grids
   cplx<R> *btiles = nullptr;  // batched spreading tiles
@@ -342,6 +380,16 @@ void launch_gather_tiles(const Engine<R> &e, cplx<R> *g, hipStream_t s, int nb =
                          const BinGeom *gb = nullptr, cplx<R> *tiles = nullptr);
 template <typename R>
 bool batch_kernels(const Engine<R> &e);
+// the same on the matrix cores (geom.mx)
+template <typename R>
+void launch_mx_interp(const cplx<R> *g, cplx<R> *f, const Engine<R> &e, hipStream_t s, int nb,
+                      const BinGeom *gb);
+template <typename R>
+void launch_mx_spread(const cplx<R> *f, const Engine<R> &e, hipStream_t s, int nb,
+                      const BinGeom *gb, cplx<R> *tiles);
+template <typename R>
+void launch_mx_gather(const Engine<R> &e, cplx<R> *g, hipStream_t s, int nb, const BinGeom *gb,
+                      cplx<R> *tiles);
 template <typename R>
 void launch_ndft(const R *x, const cplx<R> *in, cplx<R> *out, int d, const long *N, long M,
                  int adjoint, hipStream_t s);

@@ -1,0 +1,894 @@
+// B and B^T for d = 3 on the matrix cores.
+//
+// The bins are narrow enough that the taps of all their nodes fall on 16 grid
+// positions along each of the two last dimensions (bin edge at most 17 - W,
+// W = 2m + 2 taps; 7 cells at m = 4).  A node's window over those positions
+// is its W values at its offset in the bin and zeros elsewhere, and both
+// transforms become products with 16 x 16 operands:
+//
+//   B^T  T_i[e1][e2] += sum_k (psi0_k[i] psi1_k[e1]) (psi2_k[e2] f_k)
+//        for the W planes i of four nodes k of one dimension-0 cell: one
+//        16 x 16 x 4 product per plane and real / imaginary part, the tile
+//        planes staying in registers.  Nodes arrive sorted by their
+//        dimension-0 cell along a whole column of bins, so a wavefront keeps
+//        a ring of W planes and writes a plane out when the nodes have passed
+//        it: no LDS tile, no read-modify-write, no atomics.
+//   B    C[e1][k] += sum_{i, e2} g_i[e1][e2] (psi0_k[i] psi2_k[e2])
+//        for 16 nodes k: four 16 x 16 x 4 products per plane and part, then
+//        f_k = sum_e1 psi1_k[e1] C[e1][k].  A wavefront walks down the column
+//        with the planes its nodes reach in registers.
+//
+// Bound: the matrix cores and the vector ALUs together.  A node costs W planes
+// x 2 parts x 16 x 16 multiply-adds, of which (W/16)^2 meet a nonzero window:
+// at m = 4 160 cycles of a SIMD in FP32 (v_mfma_f32_16x16x4_f32, 32 cycles
+// each), 320 in FP64; vector instructions do not overlap with these (measured:
+// 5.5 cycles each between FP32 products), so the kernels are built to issue
+// few of them per node.  Measured against the LDS-tile kernels (spread_impl.hpp,
+// spread_runs.hpp), m = 4, 256^3 grid:
+//   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.70 + 0.36 (reduction)
+//   B^T, FP64, 2^21 uniform nodes     3.49 + 1.87 ms -> 0.75 + 0.60
+//   B,   FP64, 2^21 uniform nodes     7.03 ms -> 0.96
+//   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.53 (k_mx_interp3s)
+// FP64 on sparse nodes (6 per column and plane) is bound by its grid traffic:
+// 256 / 49 grid cells read or written per cell, 41 planes per 32.
+#pragma once
+
+#include "engine.hpp"
+#include "window.hpp"
+
+namespace nfft_hip {
+
+template <typename R> struct MxTypes;
+template <> struct MxTypes<float> {
+  using v4 = float __attribute__((ext_vector_type(4)));
+};
+template <> struct MxTypes<double> {
+  using v4 = double __attribute__((ext_vector_type(4)));
+};
+template <typename R> using mx4 = typename MxTypes<R>::v4;
+
+// c + a b for a 16 x 4 operand a (lane l holds row l & 15, column l >> 4), a
+// 4 x 16 operand b (lane l: row l >> 4, column l & 15) and a 16 x 16 result
+// (lane l, element r: column l & 15 and row mx_row<R>(l, r)).
+__device__ __forceinline__ mx4<float> mx_mul(float a, float b, mx4<float> c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ mx4<double> mx_mul(double a, double b, mx4<double> c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+template <typename R> __device__ __forceinline__ int mx_row(int q, int r) {
+  return sizeof(R) == 4 ? 4 * q + r : q + 4 * r;
+}
+
+// DPP move within 16-lane rows: lane I of the row
+template <int CTRL> __device__ __forceinline__ float mx_dpp(float x) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double mx_dpp(double x) {
+  const long long u = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(u & 0xffffffffLL), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+template <int I, typename R> __device__ __forceinline__ R mx_bcast(R x) {
+  return mx_dpp<0x150 + I>(x);
+}
+// sum over the four lanes of a column (l & 15), in every lane
+__device__ __forceinline__ float mx_col_sum(float x) {
+  const int v = __float_as_int(x);
+  auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  x = __int_as_float(a[0]) + __int_as_float(a[1]);
+  const int w = __float_as_int(x);
+  auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  return __int_as_float(b[0]) + __int_as_float(b[1]);
+}
+__device__ __forceinline__ double mx_col_sum(double x) {
+  x += __shfl_xor(x, 32, 64);
+  return x + __shfl_xor(x, 16, 64);
+}
+
+// Window rows of a chunk of nodes in LDS: row (t, node) holds the node's
+// dimension-t window over the positions, kMxPitch elements apart (rows of 16
+// or more positions; 20 spreads the 4 x 16 operand reads over the banks).
+constexpr int kMxPitch = 20;
+// coefficients per polynomial in the LDS table of plans whose dimensions
+// differ in sigma
+template <typename R> constexpr int kMxCoef = (poly_deg_v<R> + 4) / 4 * 4;
+
+// One window row: taps at positions shift .. shift + W - 1, zeros at the other
+// positions of the row.  Tap pairs (w, W-1-w) come from one polynomial's even
+// and odd parts at tt = frac - 1/2; pc(w) gives tap w's coefficients.
+template <typename R, int W, typename Coef>
+__device__ __forceinline__ void mx_window_row(R *row, int shift, R tt, Coef pc) {
+  constexpr int PD = poly_deg_v<R>;
+  constexpr int KE = PD - (PD % 2);      // highest even power
+  constexpr int KO = PD - 1 + (PD % 2);  // highest odd power
+  constexpr int V = 16 / sizeof(R);
+  using vec = R __attribute__((ext_vector_type(V)));
+#pragma unroll
+  for (int z = 0; z < kMxPitch; z += V) *reinterpret_cast<vec *>(row + z) = vec(0);
+  const R t2 = tt * tt;
+  R *at = row + shift;
+#pragma unroll
+  for (int w = 0; w < W / 2; w++) {
+    const R *c = pc(w);
+    R e = c[KE];
+#pragma unroll
+    for (int k = KE - 2; k >= 0; k -= 2) e = fma(e, t2, c[k]);
+    R o = c[KO];
+#pragma unroll
+    for (int k = KO - 2; k >= 1; k -= 2) o = fma(o, t2, c[k]);
+    at[w] = fma(tt, o, e);
+    at[W - 1 - w] = fma(-tt, o, e);
+  }
+}
+
+// copies the window polynomials of D dimensions (lower half of the taps) to
+// LDS, kMxCoef apart
+template <typename R, int D, int W>
+__device__ __forceinline__ void mx_load_poly(R *spoly, const R *poly, int tid, int nthr) {
+  constexpr int C = poly_deg_v<R> + 1, H = W / 2;
+  for (int i = tid; i < D * H * C; i += nthr) {
+    const int k = i % C, w = (i / C) % H, t = i / (C * H);
+    spoly[(t * H + w) * kMxCoef<R> + k] = poly[(t * W + w) * C + k];
+  }
+}
+
+// v[r] = 0 in place, for a branch of the node loop: a plain assignment made the
+// compiler copy all accumulators at the loop's head
+template <typename V> __device__ __forceinline__ void mx_clear(V &v, int r) {
+  auto x = v[r];
+  if constexpr (sizeof(x) == 4) asm("v_mov_b32 %0, 0" : "+v"(x));
+  else asm("v_mov_b64 %0, 0" : "+v"(x));
+  v[r] = x;
+}
+
+// a[i] = p1 times lane i of every 16-lane row of p0
+template <typename R, int H, int I = 0>
+__device__ __forceinline__ void mx_weights(R (&a)[H], R p0, R p1) {
+  a[I] = mx_bcast<I>(p0) * p1;
+  if constexpr (I + 1 < H) mx_weights<R, H, I + 1>(a, p0, p1);
+}
+
+// B^T of one work item: a run of nodes of one column (dimension-1 and -2
+// bins), sorted by dimension-0 cell.  Two wavefronts per item, each
+// evaluating the windows of 16 nodes of a chunk of 32 (lane = node + 16
+// dimension) into LDS and owning half of the ring's planes; both read the
+// windows back as the products' operands, four nodes of one dimension-0 cell
+// at a time (fewer where the cell's nodes or the chunk end; the missing ones
+// enter with value zero).  Output: the item's planes of 16 x 16 cells in
+// scratch, summed into the grid by k_mx_gather3.
+template <typename R, int W, bool SHARED>
+__global__ __launch_bounds__(128, sizeof(R) == 4 ? 4 : 2) void k_mx_spread3(
+    const cplx<R> *__restrict__ fin, cplx<R> *__restrict__ tiles, const int *__restrict__ perm,
+    const int *__restrict__ cell, const R *__restrict__ frac, const int4 *__restrict__ subs,
+    const int4 *__restrict__ info, BinGeom gg, WinParams<R> wp) {
+  constexpr int NC = 32, H = W / 2;
+  __shared__ __align__(16) R win[3 * NC * kMxPitch];
+  __shared__ __align__(16) cplx<R> sf[NC];
+  __shared__ int sc0[NC];
+  __shared__ __align__(16) R spoly[SHARED ? 1 : 3 * (W / 2) * kMxCoef<R>];
+  // right-hand side blockIdx.y of a batched launch
+  fin += (long)blockIdx.y * gg.bs_f;
+  tiles += (long)blockIdx.y * gg.bs_t;
+  const int4 sp = subs[blockIdx.x];
+  const int4 nf = info[sp.w];  // first plane in scratch, first node's cell, planes
+  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int me = wv * 16 + j;  // node of the chunk whose windows this lane evaluates
+  const int t = q < 3 ? q : 0;
+  const int col = sp.x / gg.nb[0];
+  const int b1 = col / gg.nb[2], b2 = col - b1 * gg.nb[2];
+  const int lo = t == 1 ? mx_lo(b1, gg.n[1], gg.nb[1]) : mx_lo(b2, gg.n[2], gg.nb[2]);
+  if constexpr (!SHARED) {
+    mx_load_poly<R, 3, W>(spoly, wp.poly, threadIdx.x, 128);
+    __syncthreads();
+  }
+  mx4<R> acc[H][2];
+#pragma unroll
+  for (int i = 0; i < H; i++) acc[i][0] = acc[i][1] = mx4<R>{0, 0, 0, 0};
+  const int *cellp = cell + t * gg.M + sp.y;
+  const R *fracp = frac + t * gg.M + sp.y;
+  const int *permp = perm + sp.y;
+  const int last = sp.z - 1;
+  // node data one chunk ahead, node indices two
+  int c = cellp[min(me, last)];
+  R fr = fracp[min(me, last)];
+  cplx<R> fv = cplx<R>{0, 0};
+  int pnext = 0;
+  if (q == 3) {
+    fv = fin[permp[min(me, last)]];
+    pnext = permp[min(NC + me, last)];
+  }
+  // the plane of a node's tap i is slot (its cell + i) mod W of the ring,
+  // slots H wv .. H wv + H - 1 in this wavefront: lane i of a 16-lane row
+  // reads the weight of own slot i, so that the products need no case per
+  // rotation
+  int a0 = nf.y;              // dimension-0 cell of the nodes at hand
+  int rot = a0 % W - H * wv;  // own slot of its first plane, which no later cell reaches
+  auto tap_of_slot = [&]() {
+    const int i = (j < H ? j : 0) - rot;
+    return i < 0 ? i + W : i;
+  };
+  int t0 = tap_of_slot();
+  cplx<R> *out = tiles + (long)nf.x * 256 + j;
+  auto flush = [&]() {
+#pragma unroll
+    for (int s = 0; s < H; s++)
+      if (rot == s) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          // (opaque copies: the compiler otherwise keeps the accumulators as
+          // (re, im) pairs across the node loop and moves all of them around
+          // every product, 40 moves per 20 of them)
+          R vr = acc[s][0][r], vi = acc[s][1][r];
+          asm("" : "+v"(vr));
+          asm("" : "+v"(vi));
+          out[mx_row<R>(q, r) * 16] = cplx<R>{vr, vi};
+          mx_clear(acc[s][0], r);
+          mx_clear(acc[s][1], r);
+        }
+      }
+    out += 256;
+    rot = rot + 1 < W - H * wv ? rot + 1 : -H * wv;
+  };
+  for (int base = 0; base < sp.z; base += NC) {
+    if (q < 3) {
+      const R *poly = wp.poly;
+      // (the coefficients are read again for every chunk: held over the
+      // loop they would take all registers)
+      asm volatile("" : "+s"(poly));
+      mx_window_row<R, W>(win + (t * NC + me) * kMxPitch, t == 0 ? 0 : c - lo, fr - R(0.5),
+                          [&](int w) {
+                            if constexpr (SHARED) return poly + w * (poly_deg_v<R> + 1);
+                            else return spoly + (t * (W / 2) + w) * kMxCoef<R>;
+                          });
+      if (q == 0) sc0[me] = c;
+    } else {
+      sf[me] = fv;
+    }
+    const int nn = min(base + NC + me, last);
+    c = cellp[nn];
+    fr = fracp[nn];
+    if (q == 3) {
+      fv = fin[pnext];
+      pnext = permp[min(base + 2 * NC + me, last)];
+    }
+    __syncthreads();
+    const int cnt = min(NC, sp.z - base);
+    const int c0 = sc0[lane & (NC - 1)];
+    for (int k = 0; k < cnt;) {
+      // the nodes k .. end - 1 of one cell
+      const int ak = __builtin_amdgcn_readlane(c0, k);
+      const unsigned long long same = __ballot(lane < cnt && c0 == ak) >> k;
+      const int end = k + (int)__builtin_ctzll(~same);
+      if (a0 < ak) {
+        for (; a0 < ak; a0++) flush();
+        t0 = tap_of_slot();
+      }
+      auto four = [&](int idx, bool live) {
+        const R *row = win + idx * kMxPitch;
+        const R p0 = row[t0], p1 = row[NC * kMxPitch + j], p2 = row[2 * NC * kMxPitch + j];
+        const cplx<R> v = sf[idx];
+        const R br = live ? p2 * v.x : R(0), bi = live ? p2 * v.y : R(0);
+        R a[H];
+        mx_weights<R, H>(a, p0, p1);
+#pragma unroll
+        for (int i = 0; i < H; i++) {
+          acc[i][0] = mx_mul(a[i], br, acc[i][0]);
+          acc[i][1] = mx_mul(a[i], bi, acc[i][1]);
+        }
+      };
+      for (; k + 4 <= end; k += 4) four(k + q, true);
+      if (k < end) four(min(k + q, NC - 1), k + q < end);
+      k = end;
+    }
+    __syncthreads();
+  }
+  for (int i = 0; i < W; i++) flush();
+}
+
+// B of one work item (the items of k_mx_spread3), 16 nodes at a time.  The
+// products' second operand is the grid: a wavefront keeps the planes that the
+// nodes at hand reach in registers, a ring of W + kMxSpan - 1 planes of which
+// a chunk's nodes of up to kMxSpan dimension-0 cells use W .. W + kMxSpan - 1,
+// and loads each plane once as the nodes move on (the next one ahead of its
+// use).  FP32: both parts in one wavefront; FP64: the real parts in one, the
+// imaginary parts in the other.
+constexpr int kMxSpan = 4;
+template <typename R> constexpr int kMxParts = sizeof(R) == 4 ? 1 : 2;
+
+template <typename R, int W, bool SHARED>
+__global__ __launch_bounds__(64 * kMxParts<R>, sizeof(R) == 4 && W <= 10 ? 3 : 2) void k_mx_interp3(
+    const cplx<R> *__restrict__ g, cplx<R> *__restrict__ fout, const int *__restrict__ perm,
+    const int *__restrict__ cell, const R *__restrict__ frac, const int4 *__restrict__ subs,
+    BinGeom gg, WinParams<R> wp) {
+  constexpr int NW = kMxParts<R>, NP = 2 / NW, NC = 16 * NW;
+  constexpr int Z = kMxSpan - 1, RW = W + Z;
+  static_assert(W + 2 * Z <= kMxPitch, "zeros before and after the dimension-0 taps");
+  // window rows: dimension 1, 0 (taps from position Z on), 2.  (A lane whose
+  // node is not of the cells at hand reads outside its dimension-0 row, at
+  // most a bin's cells away and so inside win, and drops its result.)
+  __shared__ __align__(16) R win[3 * NC * kMxPitch];
+  __shared__ int sc0[NC];
+  __shared__ __align__(16) R spoly[SHARED ? 1 : 3 * (W / 2) * kMxCoef<R>];
+  g += (long)blockIdx.y * gg.bs_g;
+  fout += (long)blockIdx.y * gg.bs_f;
+  const int4 sp = subs[blockIdx.x];
+  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+  const int wv = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int me = wv * 16 + j;
+  // dimension whose windows this lane evaluates, and its place in win
+  const int t = q < 3 ? q : 0, tp = t == 2 ? 2 : 1 - t;
+  const int col = sp.x / gg.nb[0];
+  const int b1 = col / gg.nb[2], b2 = col - b1 * gg.nb[2];
+  const int lo1 = mx_lo(b1, gg.n[1], gg.nb[1]), lo2 = mx_lo(b2, gg.n[2], gg.nb[2]);
+  const int shift0 = t == 0 ? 0 : (t == 1 ? lo1 : lo2);
+  if constexpr (!SHARED) {
+    mx_load_poly<R, 3, W>(spoly, wp.poly, threadIdx.x, 64 * NW);
+    __syncthreads();
+  }
+  // this lane's grid cells: row e1 = j, columns e2 = 4 q + s
+  long goff[4];
+  {
+    int c1 = lo1 - gg.m + j;
+    c1 += c1 < 0 ? gg.n[1] : (c1 >= gg.n[1] ? -gg.n[1] : 0);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      int c2 = lo2 - gg.m + 4 * q + s;
+      c2 += c2 < 0 ? gg.n[2] : (c2 >= gg.n[2] ? -gg.n[2] : 0);
+      goff[s] = (long)c1 * gg.n[2] + c2;
+    }
+  }
+  const long plane = (long)gg.n[1] * gg.n[2];
+  auto load_plane = [&](int p, R (&d)[NP][4]) {
+    int c0 = p - gg.m;
+    c0 += c0 < 0 ? gg.n[0] : 0;
+    c0 -= c0 >= gg.n[0] ? gg.n[0] : 0;
+    const cplx<R> *gp = g + (long)c0 * plane;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      if constexpr (NP == 2) {
+        const cplx<R> v = gp[goff[s]];
+        d[0][s] = v.x;
+        d[1][s] = v.y;
+      } else {
+        d[0][s] = reinterpret_cast<const R *>(gp + goff[s])[wv];
+      }
+    }
+  };
+  int ra = cell[sp.y];  // the ring holds planes ra .. ra + RW - 1, plane p in slot p mod RW
+  int rot = ra % RW;
+  R ring[RW][NP][4], next[NP][4];
+#pragma unroll
+  for (int s = 0; s < RW; s++) load_plane(ra + (s < rot ? s - rot + RW : s - rot), ring[s]);
+  load_plane(ra + RW, next);
+  const int *cellp = cell + t * gg.M + sp.y;
+  const R *fracp = frac + t * gg.M + sp.y;
+  const int last = sp.z - 1;
+  int c = cellp[min(me, last)];
+  R fr = fracp[min(me, last)];
+  for (int base = 0; base < sp.z; base += NC) {
+    if (q < 3) {
+      const R *poly = wp.poly;
+      asm volatile("" : "+s"(poly));  // as in k_mx_spread3
+      mx_window_row<R, W>(win + (tp * NC + me) * kMxPitch, t == 0 ? Z : c - shift0, fr - R(0.5),
+                          [&](int w) {
+                            if constexpr (SHARED) return poly + w * (poly_deg_v<R> + 1);
+                            else return spoly + (t * (W / 2) + w) * kMxCoef<R>;
+                          });
+      if (q == 0) sc0[me] = c;
+    }
+    const int nn = min(base + NC + me, last);
+    c = cellp[nn];
+    fr = fracp[nn];
+    int pj[NW];
+#pragma unroll
+    for (int h = 0; h < NW; h++)
+      pj[h] = perm[sp.y + min(base + 16 * h + j, last)];
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < NW; h++) {
+      const int cnt = min(16, sp.z - base - 16 * h);
+      const int c0 = sc0[16 * h + j];
+      const R *rows = win + 16 * h * kMxPitch;
+      R a2[4];
+#pragma unroll
+      for (int s = 0; s < 4; s++) a2[s] = rows[(2 * NC + j) * kMxPitch + 4 * q + s];
+      for (int k = 0; k < cnt;) {
+        // nodes k .. end - 1: cells ak .. az
+        const int ak = __builtin_amdgcn_readlane(c0, k);
+        const int end = __popcll(__ballot(lane < cnt && c0 <= ak + Z));
+        const int az = __builtin_amdgcn_readlane(c0, end - 1);
+        for (; ra < az - Z; ra++) {
+#pragma unroll
+          for (int s = 0; s < RW; s++)
+            if (rot == s) {
+#pragma unroll
+              for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int x = 0; x < NP; x++) ring[s][x][u] = next[x][u];
+            }
+          rot = rot + 1 < RW ? rot + 1 : 0;
+          load_plane(ra + 1 + RW, next);
+        }
+        mx4<R> acc[NP];
+#pragma unroll
+        for (int x = 0; x < NP; x++) acc[x] = mx4<R>{0, 0, 0, 0};
+        const R *w0 = rows + (NC + j) * kMxPitch + Z - c0;
+#pragma unroll
+        for (int s = 0; s < RW; s++) {
+          const int p = ra + (s < rot ? s - rot + RW : s - rot);
+          if (p >= ak && p < az + W) {
+            const R w = w0[p];
+            R a[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) a[u] = w * a2[u];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+              for (int x = 0; x < NP; x++) acc[x] = mx_mul(ring[s][x][u], a[u], acc[x]);
+          }
+        }
+        // rows e1, columns nodes: four rows in the lane, 16 over its column
+        R out[NP] = {};
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const R p1 = rows[j * kMxPitch + mx_row<R>(q, u)];
+#pragma unroll
+          for (int x = 0; x < NP; x++) out[x] = fma(acc[x][u], p1, out[x]);
+        }
+#pragma unroll
+        for (int x = 0; x < NP; x++) out[x] = mx_col_sum(out[x]);
+        if (lane >= k && lane < end) {
+          if constexpr (NP == 2) fout[pj[h]] = cplx<R>{out[0], out[1]};
+          else reinterpret_cast<R *>(fout + pj[h])[wv] = out[0];
+        }
+        k = end;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// B in FP32 on the bf16 products, whose rate is eight times that of the FP32
+// ones and which leave the vector ALUs free.  Grid values and weights are
+// split into three bf16 pieces each (8 + 8 + 8 bits: the pieces' sum is the
+// FP32 value), and the six products of pieces above 2^-24 of the largest are
+// summed in FP32: g w = gh wh + (gh wm + gm wh) + (gh wl + gm wm + gl wh).
+// One 16 x 16 x 32 product takes two of them over the 16 columns e2, so a plane
+// and part takes three; the planes are summed with the FP32 weights psi0 by the
+// vector ALUs,
+//   C[e1][k] += psi0_k[i] (sum_e2 g_i[e1][e2] psi2_k[e2]).
+using mx_bf2 = __bf16 __attribute__((ext_vector_type(2)));
+using mx_bf8 = __bf16 __attribute__((ext_vector_type(8)));
+using mx_f2 = float __attribute__((ext_vector_type(2)));
+using mx_u6 = unsigned __attribute__((ext_vector_type(6)));
+using mx_u4 = unsigned __attribute__((ext_vector_type(4)));
+
+// x = h + m + l in bf16 pieces (each rounded to nearest), two values at once
+__device__ __forceinline__ void mx_split(mx_f2 x, unsigned &h, unsigned &m, unsigned &l) {
+  const mx_bf2 a = __builtin_convertvector(x, mx_bf2);
+  mx_f2 r = x - __builtin_convertvector(a, mx_f2);
+  const mx_bf2 b = __builtin_convertvector(r, mx_bf2);
+  r = r - __builtin_convertvector(b, mx_f2);
+  const mx_bf2 c = __builtin_convertvector(r, mx_bf2);
+  h = __builtin_bit_cast(unsigned, a);
+  m = __builtin_bit_cast(unsigned, b);
+  l = __builtin_bit_cast(unsigned, c);
+}
+__device__ __forceinline__ mx4<float> mx_mul16(mx_u4 a, mx_u4 b, mx4<float> c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mx_bf8, a),
+                                                 __builtin_bit_cast(mx_bf8, b), c, 0, 0, 0);
+}
+
+// The form for dense node sets (three nodes or more per occupied cell): 32
+// nodes of up to two dimension-0 cells at a time share the ring's planes,
+// without a branch per plane.  On the 3-D kooshball 1.53 ms against 1.96 for
+// k_mx_interp3 and 1.62 for the LDS-tile kernel; on 0.09 nodes per cell
+// k_mx_interp3 is the faster one, 0.073 against 0.087 ms.  Its error against
+// 64 bits is no larger than that of FP32 products (m = 4, 64 x 64 x 64 grid:
+// 1.5e-7 against 1.7e-7), since the pieces hold all 24 bits.  The bound is the
+// issue of its 390 instructions per 16 nodes at two wavefronts per SIMD (the
+// ring takes 132 registers).
+constexpr int kMxSpanDense = 2;
+
+template <int W, bool SHARED>
+__global__ __launch_bounds__(64, 2) void k_mx_interp3s(
+    const float2 *__restrict__ g, float2 *__restrict__ fout, const int *__restrict__ perm,
+    const int *__restrict__ cell, const float *__restrict__ frac, const int4 *__restrict__ subs,
+    BinGeom gg, WinParams<float> wp) {
+  constexpr int NC = 32, Z = kMxSpanDense - 1, RW = W + Z;
+  static_assert(W + 2 * Z <= kMxPitch, "zeros before and after the dimension-0 taps");
+  __shared__ __align__(16) float win[3 * NC * kMxPitch];  // as in k_mx_interp3
+  __shared__ __align__(16) float spoly[SHARED ? 1 : 3 * (W / 2) * kMxCoef<float>];
+  g += (long)blockIdx.y * gg.bs_g;
+  fout += (long)blockIdx.y * gg.bs_f;
+  const int4 sp = subs[blockIdx.x];
+  const int lane = threadIdx.x, j = lane & 15, q = lane >> 4;
+  const int col = sp.x / gg.nb[0];
+  const int b1 = col / gg.nb[2], b2 = col - b1 * gg.nb[2];
+  const int lo1 = mx_lo(b1, gg.n[1], gg.nb[1]), lo2 = mx_lo(b2, gg.n[2], gg.nb[2]);
+  if constexpr (!SHARED) {
+    mx_load_poly<float, 3, W>(spoly, wp.poly, threadIdx.x, 64);
+    __syncthreads();
+  }
+  unsigned goff[4];
+  {
+    int c1 = lo1 - gg.m + j;
+    c1 += c1 < 0 ? gg.n[1] : (c1 >= gg.n[1] ? -gg.n[1] : 0);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      int c2 = lo2 - gg.m + 4 * q + s;
+      c2 += c2 < 0 ? gg.n[2] : (c2 >= gg.n[2] ? -gg.n[2] : 0);
+      goff[s] = (unsigned)c1 * gg.n[2] + c2;
+    }
+  }
+  const long plane = (long)gg.n[1] * gg.n[2];
+  auto load_plane = [&](int p, float2 (&d)[4]) {
+    int c0 = p - gg.m;
+    c0 += c0 < 0 ? gg.n[0] : 0;
+    c0 -= c0 >= gg.n[0] ? gg.n[0] : 0;
+    const float2 *gp = g + (long)c0 * plane;
+#pragma unroll
+    for (int s = 0; s < 4; s++) d[s] = gp[goff[s]];
+  };
+  // a plane's pieces, per part: low, high, middle pieces of e2 = 4 q .. 4 q + 3
+  mx_u6 ring[RW][2];
+  auto put = [](mx_u6 &r, float a, float b, float c, float d) {
+    unsigned h0, m0, l0, h1, m1, l1;
+    mx_split(mx_f2{a, b}, h0, m0, l0);
+    mx_split(mx_f2{c, d}, h1, m1, l1);
+    r = mx_u6{l0, l1, h0, h1, m0, m1};
+  };
+  auto put_plane = [&](mx_u6 (&r)[2], const float2 (&d)[4]) {
+    put(r[0], d[0].x, d[1].x, d[2].x, d[3].x);
+    put(r[1], d[0].y, d[1].y, d[2].y, d[3].y);
+  };
+  int ra = cell[sp.y];  // the ring holds planes ra .. ra + RW - 1, plane p in slot p mod RW
+  int rot = ra % RW;
+  float2 next[4];
+#pragma unroll
+  for (int s = 0; s < RW; s++) {
+    float2 d[4];
+    load_plane(ra + (s < rot ? s - rot + RW : s - rot), d);
+    put_plane(ring[s], d);
+  }
+  load_plane(ra + RW, next);
+  // lane = node + 32 t evaluates dimension t = 0, 1 and, lanes below 32,
+  // dimension 2 (rows of win: dimension 1, 0, 2)
+  const int me = lane & 31, t = lane >> 5;
+  const int *cellp = cell + t * gg.M + sp.y, *cell2 = cell + 2 * gg.M + sp.y;
+  const float *fracp = frac + t * gg.M + sp.y, *frac2 = frac + 2 * gg.M + sp.y;
+  const int *permp = perm + sp.y;
+  const int last = sp.z - 1;
+  int c = cellp[min(me, last)], d2 = cell2[min(me, last)];
+  float fr = fracp[min(me, last)], fr2 = frac2[min(me, last)];
+  for (int base = 0; base < sp.z; base += NC) {
+    const int c0 = c;  // lanes 0..31: the chunk's dimension-0 cells
+    {
+      const float *poly = wp.poly;
+      asm volatile("" : "+s"(poly));  // as in k_mx_spread3
+      mx_window_row<float, W>(win + ((1 - t) * NC + me) * kMxPitch, t == 0 ? Z : c - lo1, fr - 0.5f,
+                              [&](int w) {
+                                if constexpr (SHARED) return poly + w * (kPolyDeg + 1);
+                                else return spoly + (t * (W / 2) + w) * kMxCoef<float>;
+                              });
+      if (t == 0)
+        mx_window_row<float, W>(win + (2 * NC + me) * kMxPitch, d2 - lo2, fr2 - 0.5f, [&](int w) {
+          if constexpr (SHARED) return poly + w * (kPolyDeg + 1);
+          else return spoly + (W + w) * kMxCoef<float>;
+        });
+    }
+    const int pj = permp[min(base + me, last)];
+    const int nn = min(base + NC + me, last);
+    c = cellp[nn];
+    fr = fracp[nn];
+    d2 = cell2[nn];
+    fr2 = frac2[nn];
+    __syncthreads();
+    const int cnt = min(NC, sp.z - base);
+    // weights of the nodes j and j + 16 for the piece pairs (h, m), (l, h), (h, m)
+    mx_u4 w1[2], w2[2], w3[2];
+    int cj[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const float *r2 = win + (2 * NC + 16 * h + j) * kMxPitch + 4 * q;
+      unsigned h0, m0, l0, h1, m1, l1;
+      mx_split(mx_f2{r2[0], r2[1]}, h0, m0, l0);
+      mx_split(mx_f2{r2[2], r2[3]}, h1, m1, l1);
+      w1[h] = mx_u4{h0, h1, h0, h1};
+      w2[h] = mx_u4{h0, h1, m0, m1};
+      w3[h] = mx_u4{l0, l1, m0, m1};
+      cj[h] = __shfl(c0, 16 * h + j, 64);
+    }
+    for (int k = 0; k < cnt;) {
+      // nodes k .. end - 1: cells ak .. az
+      const int ak = __builtin_amdgcn_readlane(c0, k);
+      const int end = __popcll(__ballot(lane < cnt && c0 <= ak + Z));
+      const int az = __builtin_amdgcn_readlane(c0, end - 1);
+      for (; ra < az - Z; ra++) {
+        mx_u6 nx[2];
+        put_plane(nx, next);
+#pragma unroll
+        for (int s = 0; s < RW; s++)
+          if (rot == s) {
+            ring[s][0] = nx[0];
+            ring[s][1] = nx[1];
+          }
+        rot = rot + 1 < RW ? rot + 1 : 0;
+        load_plane(ra + 1 + RW, next);
+      }
+      // planes that a node does not reach meet zeros of its row (ra <= ak and
+      // ra + Z >= az)
+      mx4<float> acc[2][2] = {};
+      const float *w0[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        w0[h] = win + (NC + 16 * h + j) * kMxPitch + Z - cj[h] + ra;
+#pragma unroll
+      for (int s = 0; s < RW; s++) {
+        const int i = s < rot ? s - rot + RW : s - rot;
+        mx_u4 a[2], b[2];
+#pragma unroll
+        for (int x = 0; x < 2; x++) {
+          b[x] = __builtin_shufflevector(ring[s][x], ring[s][x], 0, 1, 2, 3);
+          a[x] = __builtin_shufflevector(ring[s][x], ring[s][x], 2, 3, 4, 5);
+        }
+        mx4<float> z[2][2] = {};
+        // small products first
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int x = 0; x < 2; x++) z[h][x] = mx_mul16(a[x], w3[h], z[h][x]);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int x = 0; x < 2; x++) z[h][x] = mx_mul16(b[x], w2[h], z[h][x]);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int x = 0; x < 2; x++) z[h][x] = mx_mul16(a[x], w1[h], z[h][x]);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          const float w = w0[h][i];
+#pragma unroll
+          for (int x = 0; x < 2; x++)
+#pragma unroll
+            for (int u = 0; u < 4; u++) acc[h][x][u] = fmaf(w, z[h][x][u], acc[h][x][u]);
+        }
+      }
+      float out[2][2] = {};
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const float p1 = win[(16 * h + j) * kMxPitch + 4 * q + u];
+#pragma unroll
+          for (int x = 0; x < 2; x++) out[h][x] = fmaf(acc[h][x][u], p1, out[h][x]);
+        }
+#pragma unroll
+        for (int x = 0; x < 2; x++) out[h][x] = mx_col_sum(out[h][x]);
+      }
+      // lanes 0..31: node = lane
+      if (lane >= k && lane < end)
+        fout[pj] = float2{lane < 16 ? out[0][0] : out[1][0], lane < 16 ? out[0][1] : out[1][1]};
+      k = end;
+    }
+    __syncthreads();
+  }
+}
+
+// Sums the planes of the items of a spreading bin that has several (dense
+// bins, up to hundreds of items) into one tile of the bin's planes, so that
+// the reduction below reads one tile per bin.  A workgroup owns one plane of
+// one such bin; a thread one cell.
+template <typename R>
+__global__ __launch_bounds__(256) void k_mx_sum3(cplx<R> *__restrict__ tiles,
+                                                 const int4 *__restrict__ info,
+                                                 const int4 *__restrict__ bin_info,
+                                                 const int *__restrict__ multi,
+                                                 const int *__restrict__ sp_first,
+                                                 const int *__restrict__ sp_count, BinGeom gg) {
+  tiles += (long)blockIdx.z * gg.bs_t;
+  const int bin = multi[blockIdx.x];
+  const int4 bi = bin_info[bin];  // first plane in scratch, dimension-0 cell, planes
+  const int pl = blockIdx.y;
+  if (pl >= bi.z) return;
+  const int first = sp_first[bin], cnt = sp_count[bin];
+  __shared__ int list[256];  // first to last: planes of the items that cover this one
+  __shared__ int wsum[4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  R ar = 0, ai = 0;
+  for (int s0 = 0; s0 < cnt; s0 += 256) {
+    const int s = s0 + threadIdx.x;
+    int at = -1;
+    if (s < cnt) {
+      const int4 nf = info[first + s];
+      const int p = pl - (nf.y - bi.y);
+      if (p >= 0 && p < nf.z) at = nf.x + p;
+    }
+    const unsigned long long in = __ballot(at >= 0);
+    if (lane == 0) wsum[wv] = __popcll(in);
+    __syncthreads();
+    int k = __popcll(in & ((1ull << lane) - 1));
+    for (int w = 0; w < wv; w++) k += wsum[w];
+    if (at >= 0) list[k] = at;
+    const int n = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    __syncthreads();
+    for (int i = 0; i < n; i += 8) {
+      cplx<R> v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        v[u] = i + u < n ? tiles[(long)list[i + u] * 256 + threadIdx.x] : cplx<R>{0, 0};
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        ar += v[u].x;
+        ai += v[u].y;
+      }
+    }
+    __syncthreads();
+  }
+  tiles[((long)bi.x + pl) * 256 + threadIdx.x] = cplx<R>{ar, ai};
+}
+
+// Tile reduction: every grid cell as the sum of the bins' planes that cover
+// it.  A workgroup owns one plane c0 and one dimension-1 bin's rows and up to
+// 256 cells of dimension 2; a thread owns one dimension-2 cell of all those
+// rows.  Tile rows of 16 cells are read whole by one workgroup, so each tile
+// plane is read by the three workgroups of its dimension-1 neighbourhood
+// only; these are adjacent in the launch order of one XCD and meet in its L2.
+template <typename R, int W>
+__global__ __launch_bounds__(256) void k_mx_gather3(const cplx<R> *__restrict__ tiles,
+                                                    const int4 *__restrict__ bin_info,
+                                                    cplx<R> *__restrict__ g, BinGeom gg,
+                                                    int chunks, int total) {
+  constexpr int ROWS = 17 - W;
+  tiles += (long)blockIdx.y * gg.bs_t;
+  g += (long)blockIdx.y * gg.bs_g;
+  // consecutive work of one XCD is consecutive in (plane, bin)
+  const int per = (total + 7) / 8;
+  int w = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || w >= total) return;
+  const int ch = w % chunks;
+  w /= chunks;
+  const int b1 = w % gg.nb[1], c0 = w / gg.nb[1];
+  const int n0 = gg.n[0], n1 = gg.n[1], n2 = gg.n[2];
+  const int nb1 = gg.nb[1], nb2 = gg.nb[2], nb0 = gg.nb[0];
+  const int c2 = ch * 256 + threadIdx.x;
+  if (c2 >= n2) return;
+  const int lo1 = mx_lo(b1, n1, nb1), rows = mx_lo(b1 + 1, n1, nb1) - lo1;
+  const int b2 = mx_bin(c2, n2, nb2);
+  const int bB = c0 / gg.bs[0];
+  const int s1 = gg.mx_span[1], s2 = gg.mx_span[2], s0 = gg.mx_span[0];
+  // neighbour jj of span: all bins, or the bins around the own one
+  auto nbr = [](int b, int jj, int span, int nb) {
+    if (span == nb) return jj;
+    int v = b + jj - span / 2;
+    v += v < 0 ? nb : 0;
+    return v >= nb ? v - nb : v;
+  };
+  R ar[ROWS], ai[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; i++) ar[i] = ai[i] = R(0);
+  for (int j1 = 0; j1 < s1; j1++) {
+    const int bb1 = nbr(b1, j1, s1, nb1);
+    int e1 = lo1 - mx_lo(bb1, n1, nb1) + gg.m;  // tile row of the first owned row
+    e1 += e1 < 0 ? n1 : (e1 >= n1 ? -n1 : 0);
+    for (int j0 = 0; j0 < s0; j0++) {
+      const int bb0 = nbr(bB, j0, s0, nb0);
+      // planes of that bin: none beyond its cells' windows
+      const int f0 = bb0 * gg.bs[0], h0 = min(n0, f0 + gg.bs[0]) - f0;
+      int d0 = c0 - f0 + gg.m;
+      d0 += d0 < 0 ? n0 : (d0 >= n0 ? -n0 : 0);
+      if (d0 >= h0 + W - 1) continue;
+      for (int j2 = 0; j2 < s2; j2++) {
+        const int bb2 = nbr(b2, j2, s2, nb2);
+        int e2 = c2 - mx_lo(bb2, n2, nb2) + gg.m;
+        e2 += e2 < 0 ? n2 : (e2 >= n2 ? -n2 : 0);
+        if (e2 >= 16) continue;
+        const int4 bi = bin_info[(bb1 * nb2 + bb2) * nb0 + bb0];
+        int pl = c0 - bi.y + gg.m;
+        pl += pl < 0 ? n0 : (pl >= n0 ? -n0 : 0);
+        if (pl >= bi.z) continue;
+        const cplx<R> *tp = tiles + ((long)bi.x + pl) * 256 + e2;
+#pragma unroll
+        for (int i = 0; i < ROWS; i++) {
+          int e = e1 + i;
+          e -= e >= n1 ? n1 : 0;
+          if (e < 16 && i < rows) {
+            const cplx<R> v = tp[e * 16];
+            ar[i] += v.x;
+            ai[i] += v.y;
+          }
+        }
+      }
+    }
+  }
+  cplx<R> *gp = g + ((long)c0 * n1 + lo1) * n2 + c2;
+#pragma unroll
+  for (int i = 0; i < ROWS; i++)
+    if (i < rows) gp[(long)i * n2] = cplx<R>{ar[i], ai[i]};
+}
+
+// ==================================================================== dispatch
+template <typename R, int M_>
+void mx_spread3(const cplx<R> *f, cplx<R> *tiles, const Engine<R> &e, const BinGeom &gg,
+                hipStream_t s, int nb) {
+  auto fn = e.win.poly_shared ? k_mx_spread3<R, 2 * M_ + 2, true> : k_mx_spread3<R, 2 * M_ + 2, false>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)e.sp_nsub, (unsigned)nb), dim3(128), 0, s, f,
+                     tiles, e.perm, e.cell, e.frac, e.sp_subs, e.mx_info, gg, e.win);
+}
+
+template <typename R, int M_>
+void mx_interp3(const cplx<R> *g, cplx<R> *f, const Engine<R> &e, const BinGeom &gg,
+                hipStream_t s, int nb) {
+  constexpr int W = 2 * M_ + 2;
+  if constexpr (sizeof(R) == 4) {
+    if (e.mx_dense) {
+      auto fn = e.win.poly_shared ? k_mx_interp3s<W, true> : k_mx_interp3s<W, false>;
+      hipLaunchKernelGGL(fn, dim3((unsigned)e.nsub, (unsigned)nb), dim3(64), 0, s, g, f, e.perm,
+                         e.cell, e.frac, e.subs, gg, e.win);
+      return;
+    }
+  }
+  auto fn = e.win.poly_shared ? k_mx_interp3<R, W, true> : k_mx_interp3<R, W, false>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)e.nsub, (unsigned)nb), dim3(64 * kMxParts<R>), 0, s, g, f,
+                     e.perm, e.cell, e.frac, e.subs, gg, e.win);
+}
+
+template <typename R, int M_>
+void mx_gather3(const cplx<R> *tiles, cplx<R> *g, const Engine<R> &e, const BinGeom &gg,
+                hipStream_t s, int nb) {
+  if (e.mx_multi_n > 0)
+    hipLaunchKernelGGL((k_mx_sum3<R>),
+                       dim3((unsigned)e.mx_multi_n, (unsigned)(gg.bs[0] + 2 * M_ + 1), (unsigned)nb),
+                       dim3(256), 0, s, const_cast<cplx<R> *>(tiles), e.mx_info, e.mx_bin_info,
+                       e.mx_multi, e.sp_first, e.sp_count, gg);
+  const int chunks = (gg.n[2] + 255) / 256;
+  const int total = gg.n[0] * gg.nb[1] * chunks;
+  const unsigned blocks = 8u * (unsigned)((total + 7) / 8);
+  hipLaunchKernelGGL((k_mx_gather3<R, 2 * M_ + 2>), dim3(blocks, (unsigned)nb), dim3(256), 0, s,
+                     tiles, e.mx_bin_info, g, gg, chunks, total);
+}
+
+// the launches of window cut-off m (1 .. kMxMaxM)
+#define NFFT_MX_DISPATCH(FN, ...)              \
+  switch (gg.m) {                              \
+    case 1: FN<R, 1>(__VA_ARGS__); break;      \
+    case 2: FN<R, 2>(__VA_ARGS__); break;      \
+    case 3: FN<R, 3>(__VA_ARGS__); break;      \
+    case 4: FN<R, 4>(__VA_ARGS__); break;      \
+    case 5: FN<R, 5>(__VA_ARGS__); break;      \
+    case 6: FN<R, 6>(__VA_ARGS__); break;      \
+    default: break;                            \
+  }
+
+template <typename R>
+void launch_mx_spread(const cplx<R> *f, const Engine<R> &e, hipStream_t s, int nb,
+                      const BinGeom *gb, cplx<R> *tiles) {
+  if (e.sp_nsub == 0) return;
+  const BinGeom &gg = gb ? *gb : e.geom;
+  if (!tiles) tiles = e.tiles;
+  NFFT_MX_DISPATCH(mx_spread3, f, tiles, e, gg, s, nb)
+}
+
+template <typename R>
+void launch_mx_interp(const cplx<R> *g, cplx<R> *f, const Engine<R> &e, hipStream_t s, int nb,
+                      const BinGeom *gb) {
+  if (e.nsub == 0) return;
+  const BinGeom &gg = gb ? *gb : e.geom;
+  NFFT_MX_DISPATCH(mx_interp3, g, f, e, gg, s, nb)
+}
+
+template <typename R>
+void launch_mx_gather(const Engine<R> &e, cplx<R> *g, hipStream_t s, int nb, const BinGeom *gb,
+                      cplx<R> *tiles) {
+  const BinGeom &gg = gb ? *gb : e.geom;
+  if (!tiles) tiles = e.tiles;
+  NFFT_MX_DISPATCH(mx_gather3, tiles, g, e, gg, s, nb)
+}
+#undef NFFT_MX_DISPATCH
+
+}  // namespace nfft_hip

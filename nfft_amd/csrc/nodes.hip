@@ -32,7 +32,7 @@ __global__ void k_node_prep(const R *__restrict__ x, BinGeom gg, int cap,
                             int *__restrict__ key_of, int *__restrict__ khist) {
   long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= gg.M) return;
-  int bin = 0, local = 0;
+  int bin = 0, local = 0, bin0 = 0;
   for (int t = 0; t < gg.d; t++) {
     double y = (double)x[j * gg.d + t] * (double)gg.n[t];
     double c = floor(y);
@@ -41,10 +41,20 @@ __global__ void k_node_prep(const R *__restrict__ x, BinGeom gg, int cap,
     if (cw < 0) cw += gg.n[t];
     cell_tmp[t * gg.M + j] = (int)cw;
     frac_tmp[t * gg.M + j] = (R)fr;
+    if (gg.mx && t > 0) {
+      // ragged bins
+      const int bt = mx_bin((int)cw, gg.n[t], gg.nb[t]);
+      bin = bin * gg.nb[t] + bt;
+      local = local * gg.bs[t] + ((int)cw - mx_lo(bt, gg.n[t], gg.nb[t]));
+      continue;
+    }
     const int bt = (int)cw / gg.bs[t];
-    bin = bin * gg.nb[t] + bt;
+    if (gg.mx) bin0 = bt;
+    else bin = bin * gg.nb[t] + bt;
     local = local * gg.bs[t] + ((int)cw - bt * gg.bs[t]);
   }
+  // matrix-core plans number their bins with dimension 0 fastest
+  if (gg.mx) bin = bin * gg.nb[0] + bin0;
   const int key = bin * cap + local;
   key_of[j] = key;
   atomicAdd(&khist[key], 1);
@@ -144,6 +154,87 @@ __global__ void k_bins_from_keys(const int *__restrict__ kstart, long nbins, int
   const int next = b + 1 < nbins ? kstart[(b + 1) * cap] : total;
   bin_start[b] = first;
   hist[b] = next - first;
+}
+
+// occupied cells: positions where the sorted key changes
+__global__ __launch_bounds__(256) void k_count_cells(const unsigned *__restrict__ key, long M,
+                                                     int *__restrict__ count) {
+  const long j = (long)blockIdx.x * 256 + threadIdx.x;
+  const int n = __popcll(__ballot(j < M && (j == 0 || key[j] != key[j - 1])));
+  __shared__ int sum[4];
+  if ((threadIdx.x & 63) == 0) sum[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(count, sum[0] + sum[1] + sum[2] + sum[3]);
+}
+
+// Planes of every spreading item of a matrix-core plan (items in bin order):
+// from its first node's dimension-0 cell to its last node's, W - 1 more
+__global__ void k_mx_planes(const int4 *__restrict__ items, long nitems,
+                            const int *__restrict__ cell0, int W, int *__restrict__ planes) {
+  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nitems) return;
+  const int4 it = items[i];
+  planes[i] = cell0[it.y + it.z - 1] - cell0[it.y] + W;
+}
+__global__ void k_mx_info(const int4 *__restrict__ items, long nitems,
+                          const int *__restrict__ cell0, const int *__restrict__ planes,
+                          const int *__restrict__ plane_off, int4 *__restrict__ info) {
+  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nitems) return;
+  info[i] = make_int4(plane_off[i], cell0[items[i].y], planes[i], 0);
+}
+// Per spreading bin the planes the tile reduction reads (see Engine); bins of
+// several items are listed and get a tile of their own behind the items',
+// *item_planes planes into scratch
+__global__ void k_mx_bin_info(const int *__restrict__ sp_first, const int *__restrict__ sp_count,
+                              long nbins, BinGeom gg, const int4 *__restrict__ info,
+                              const int *__restrict__ item_planes, int *__restrict__ nmulti,
+                              int *__restrict__ multi, int4 *__restrict__ bin_info) {
+  long b = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nbins) return;
+  const int cnt = sp_count[b];
+  int4 v = make_int4(0, 0, 0, 0);
+  if (cnt == 1) v = info[sp_first[b]];
+  if (cnt > 1) {
+    const int f0 = (int)(b % gg.nb[0]) * gg.bs[0];
+    const int k = atomicAdd(nmulti, 1);
+    multi[k] = (int)b;
+    const int full = gg.bs[0] + 2 * gg.m + 1;
+    v = make_int4(*item_planes + k * full, f0, min(gg.n[0] - f0, gg.bs[0]) + 2 * gg.m + 1, 0);
+  }
+  bin_info[b] = v;
+}
+
+// Spreading items that the bins of the LDS-tile kernels would give a
+// matrix-core plan's nodes: a histogram over those bins (lanes of one bin
+// add once), then the items of every bin.
+__global__ void k_tile_bin_hist(const int *__restrict__ cell, BinGeom tg, int *__restrict__ hist) {
+  const long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  int bin = -1;
+  if (j < tg.M) {
+    bin = 0;
+    for (int t = 0; t < tg.d; t++) bin = bin * tg.nb[t] + cell[t * tg.M + j] / tg.bs[t];
+  }
+  while (__any(bin >= 0)) {
+    const unsigned long long left = __ballot(bin >= 0);
+    const int lead = __ffsll(left) - 1;
+    const int b = __shfl(bin, lead, 64);
+    const unsigned long long same = __ballot(bin == b);
+    if (bin == b) {
+      if ((int)(threadIdx.x & 63) == lead) atomicAdd(&hist[b], __popcll(same));
+      bin = -1;
+    }
+  }
+}
+__global__ __launch_bounds__(256) void k_tile_items(const int *__restrict__ hist, long nbins,
+                                                    int max_per_sub, int max_items,
+                                                    int *__restrict__ sum) {
+  int s = 0;
+  for (long b = threadIdx.x; b < nbins; b += 256) s += items_of(hist[b], max_per_sub, max_items);
+  __shared__ int sh[256];
+  int total;
+  block_exclusive_sum_256(s, sh, total);
+  if (threadIdx.x == 0) *sum = total;
 }
 
 // sorted position p holds node order[p]: its index and its cell / frac
@@ -412,7 +503,13 @@ void bin_nodes(Engine<R> &e) {
   const long b_keys = al(nkeys * (long)sizeof(int));
   // the tile sums also serve scans of M-long node arrays
   const long b_tiles = al(std::max(ntiles, ceil_div(M + 1, kScanTile)) * (long)sizeof(int));
-  const long b_bins = al(nbins * (long)sizeof(int));
+  // the bins of the LDS-tile kernels a matrix-core plan would otherwise use
+  long ntbins = 0;
+  if (gg.mx && e.tile_batchable) {
+    ntbins = 1;
+    for (int t = 0; t < gg.d; t++) ntbins *= e.tile_geom.nb[t];
+  }
+  const long b_bins = al(std::max(nbins, ntbins) * (long)sizeof(int));
   const long b_M = al(M * (long)sizeof(int));
   const long b_cell = al((long)gg.d * M * (long)sizeof(int));
   const long b_frac = al((long)gg.d * M * (long)sizeof(R));
@@ -511,10 +608,23 @@ void bin_nodes(Engine<R> &e) {
     }
   };
   make_list(e.max_per_sub, 0, sub_start, nsub_of, &e.subs, &e.subs_cap, &e.nsub);
+  // Dense node sets of FP32 matrix-core plans: three nodes or more per
+  // occupied cell, where k_mx_interp3s is the faster B kernel (mx.hpp; the
+  // kooshball holds 5.3)
+  e.mx_dense = false;
+  if (gg.mx && sizeof(R) == 4 && M > 0) {
+    int cells = 0;
+    launch_fill_zero_int(sums + 1, 1, s);
+    hipLaunchKernelGGL(k_count_cells, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s, key_sorted,
+                       M, sums + 1);
+    NFFT_HIP_CHECK(R, hipMemcpyAsync(&cells, sums + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+    NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
+    e.mx_dense = M >= 3L * cells;
+  }
   // interpolation slots (pairs of same-cell nodes) for the kernels that use them
   e.geom.slots = e.geom.islots = nullptr;
   e.nslots = 0;
-  if (e.use_slots() && M > 0 && e.nsub > 0) {
+  if (!gg.mx && e.use_slots() && M > 0 && e.nsub > 0) {
     auto long_scan = [&](const int *in, int *out, long len, int *total) {
       const long nt = ceil_div(len, kScanTile);
       hipLaunchKernelGGL(k_scan_tile_sums, dim3((unsigned)nt), dim3(256), 0, s, in, len, tile_sum);
@@ -584,6 +694,50 @@ void bin_nodes(Engine<R> &e) {
   e.bin_order = e.sp_first + 2 * nbins;
   make_list(e.spread_max_per_sub, e.spread_max_items, e.sp_first, e.sp_count, &e.sp_subs,
             &e.sp_subs_cap, &e.sp_nsub);
+  if (gg.mx) {
+    // the items' planes and their places in scratch (item counts are at most
+    // M, so the node-length temporaries hold them), and what the LDS-tile
+    // kernels would have needed
+    // sums + 1: item planes, bins of several items, LDS-tile items
+    int totals[3] = {0, 0, 0};
+    if (nbins > e.mx_bins_cap) {
+      if (e.mx_bin_info) NFFT_HIP_CHECK(R, hipFree(e.mx_bin_info));
+      NFFT_HIP_CHECK(R, hipMalloc(&e.mx_bin_info, (sizeof(int4) + sizeof(int)) * (size_t)nbins));
+      e.mx_multi = reinterpret_cast<int *>(e.mx_bin_info + nbins);
+      e.mx_bins_cap = nbins;
+    }
+    if (e.sp_nsub > 0) {
+      const int4 *items = e.sp_subs + e.sp_nsub;  // in bin order
+      const unsigned gi = (unsigned)ceil_div(e.sp_nsub, 256);
+      if (e.sp_nsub > e.mx_info_cap) {
+        if (e.mx_info) NFFT_HIP_CHECK(R, hipFree(e.mx_info));
+        NFFT_HIP_CHECK(R, hipMalloc(&e.mx_info, sizeof(int4) * (size_t)e.sp_nsub));
+        e.mx_info_cap = e.sp_nsub;
+      }
+      launch_fill_zero_int(sums + 1, 3, s);
+      hipLaunchKernelGGL(k_mx_planes, dim3(gi), dim3(256), 0, s, items, e.sp_nsub, e.cell,
+                         2 * gg.m + 2, key_of);
+      hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, key_of, rank_of, e.sp_nsub,
+                         sums + 1);
+      hipLaunchKernelGGL(k_mx_info, dim3(gi), dim3(256), 0, s, items, e.sp_nsub, e.cell, key_of,
+                         rank_of, e.mx_info);
+      hipLaunchKernelGGL(k_mx_bin_info, dim3((unsigned)ceil_div(nbins, 256)), dim3(256), 0, s,
+                         e.sp_first, e.sp_count, nbins, e.geom, e.mx_info, sums + 1, sums + 2,
+                         e.mx_multi, e.mx_bin_info);
+      if (ntbins > 0) {
+        launch_fill_zero_int(hist, ntbins, s);
+        hipLaunchKernelGGL(k_tile_bin_hist, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s,
+                           e.cell, e.tile_geom, hist);
+        hipLaunchKernelGGL(k_tile_items, dim3(1), dim3(256), 0, s, hist, ntbins,
+                           e.tile_spread_max_per_sub, e.spread_max_items, sums + 3);
+      }
+      NFFT_HIP_CHECK(R, hipMemcpyAsync(totals, sums + 1, 3 * sizeof(int), hipMemcpyDeviceToHost, s));
+      NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
+    }
+    e.mx_multi_n = totals[1];
+    e.tile_cells = (totals[0] + (long)totals[1] * (gg.bs[0] + 2 * gg.m + 1)) * 256L;
+    e.tile_items = totals[2];
+  }
   // heavy bins first for the zone reduction (the interpolation list's
   // temporaries are free again: bucket per bin, bucket histogram and offsets)
   if (gg.zoned) {

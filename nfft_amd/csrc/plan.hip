@@ -374,6 +374,66 @@ void Engine<R>::set_bins(const int *bs) {
   }
 }
 
+// Bins of the matrix-core B and B^T (mx.hpp) in place of the ones set by
+// set_bins, where those kernels cover the plan: d = 3, windows of up to
+// 2 kMxMaxM + 2 taps, at least 16 cells along dimensions 1 and 2 (a tile row
+// must not wrap onto itself), and no NFFT_HIP_* variable that picks an
+// LDS-tile kernel or its bins.
+template <typename R>
+void Engine<R>::set_mx_bins() {
+  const int W = 2 * m + 2;
+  if (d != 3 || m < 1 || m > kMxMaxM) return;
+  for (const char *v : {"NFFT_HIP_SPREAD", "NFFT_HIP_INTERP", "NFFT_HIP_BINS", "NFFT_HIP_ITEM",
+                        "NFFT_HIP_SPREAD_ITEM", "NFFT_HIP_SPREAD_CAP", "NFFT_HIP_ZONES",
+                        "NFFT_HIP_PAIRS", "NFFT_HIP_SLOT", "NFFT_HIP_SLOTSORT", "NFFT_HIP_SYMWIN",
+                        "NFFT_HIP_IPITCH", "NFFT_HIP_IPLANE"})
+    if (std::getenv(v)) return;
+  for (int t = 1; t < d; t++)
+    if (n[t] < 16 || n[t] > kMxMaxN) return;
+  if (n[0] > kMxMaxN) return;
+  BinGeom gg = geom;
+  gg.mx = 1;
+  gg.zoned = 0;
+  gg.zmap = gg.zdesc = nullptr;
+  long nkeys = 1;
+  for (int t = 1; t < d; t++) {
+    gg.nb[t] = (int)ceil_div(n[t], 17 - W);
+    gg.bs[t] = (int)ceil_div(n[t], gg.nb[t]);
+    // bins whose windows reach a bin's cells: the smallest bin has
+    // floor(n / nb) cells, the windows m + 1 cells beyond their bin
+    gg.mx_span[t] = std::min(gg.nb[t], 2 * (1 + m / (int)(n[t] / gg.nb[t])) + 1);
+    nkeys *= (long)gg.nb[t] * gg.bs[t];
+  }
+  // dimension 0: bins of 8 cells, 16 or 32 while at least 4096 bins remain, so
+  // that the W - 1 planes past a bin's cells weigh less (a tile must not wrap
+  // onto itself either)
+  gg.bs[0] = (int)std::min<long>(8, n[0] - W + 1);
+  for (int r : {16, 32})
+    if (r + W - 1 <= n[0] && (long)gg.nb[1] * gg.nb[2] * ceil_div(n[0], r) >= 4096) gg.bs[0] = r;
+  gg.nb[0] = (int)ceil_div(n[0], gg.bs[0]);
+  const long last = n[0] - (long)(gg.nb[0] - 1) * gg.bs[0];
+  gg.mx_span[0] = std::min(gg.nb[0], 2 * (1 + m / (int)std::min<long>(last, gg.bs[0])) + 1);
+  nkeys *= (long)gg.nb[0] * gg.bs[0];
+  if (nkeys > 0x7fffffffL) return;
+  for (int t = 0; t < d; t++) gg.E[t] = t == 0 ? gg.bs[0] + W - 1 : 16;
+  tile_geom = geom;
+  tile_batchable = batch_kernels<R>(*this);
+  tile_spread_max_per_sub = spread_max_per_sub;
+  if (zone_tab) NFFT_HIP_CHECK(R, hipFree(zone_tab));
+  zone_tab = nullptr;
+  geom = gg;
+  tile_scratch = true;
+  // nodes per item: up to 2048 (B) and 4096 (B^T, whose two wavefronts share an
+  // item and whose tiles are reduced), fewer while that leaves less than 2048
+  // items; larger ones end the launch late, smaller ones load and write more
+  // planes (3-D kooshball: B 1.65, 1.55, 1.53 ms with 512, 1024, 2048 nodes;
+  // the reduction 0.73, 0.61, 0.44, 0.37 ms with 512 to 4096)
+  max_per_sub = 2048;
+  spread_max_per_sub = 4096;
+  while (max_per_sub > 256 && max_per_sub * 2048L > M) max_per_sub /= 2;
+  while (spread_max_per_sub > 512 && spread_max_per_sub * 2048L > M) spread_max_per_sub /= 2;
+}
+
 template <typename R>
 void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) {
   d = d_;
@@ -512,6 +572,8 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
   // split by row parity; 2-D: one wavefront per tile; 1-D: private tiles);
   // double: wavefronts sharing a tile with ds_add_f64
   spread_variant = variant("NFFT_HIP_SPREAD", sizeof(R) == 4 ? (d == 3 ? 10 : (d == 2 ? 14 : 2)) : 1);
+
+  set_mx_bins();
 
   // FFT: twiddles per dimension, then the pruned passes of both directions.
   // An axis whose lines fit one workgroup's LDS (cap elements) and whose
@@ -715,6 +777,8 @@ void Engine<R>::destroy() {
   hipFree(slots);
   hipFree(slots_raw);
   hipFree(islots);
+  hipFree(mx_info);
+  hipFree(mx_bin_info);
   for (auto &e : ev)
     if (e) hipEventDestroy(e);
   for (auto &set : log_ev)
@@ -736,7 +800,8 @@ void Engine<R>::build_nodes() {
     if (tile_scratch) {
       long tot = 1;
       for (int t = 0; t < d; t++) tot *= geom.E[t];
-      const long need = sp_nsub * tot;
+      if (!geom.mx) tile_cells = sp_nsub * tot;
+      const long need = tile_cells;
       if (need > tiles_cap) {
         if (tiles) NFFT_HIP_CHECK(R, hipFree(tiles));
         NFFT_HIP_CHECK(R, hipMalloc(&tiles, sizeof(cplx<R>) * (size_t)(need > 0 ? need : 1)));
@@ -811,9 +876,7 @@ bool Engine<R>::batchable() const {
 // launch stay below 4 GiB
 template <typename R>
 int Engine<R>::batch_chunk(int nrhs) const {
-  long tot = 1;
-  for (int t = 0; t < d; t++) tot *= geom.E[t];
-  const long per_rhs = (n_total + sp_nsub * tot) * (long)sizeof(cplx<R>);
+  const long per_rhs = (n_total + tile_cells) * (long)sizeof(cplx<R>);
   const long cap = std::max(1L, (4L << 30) / std::max(1L, per_rhs));
   return (int)std::min<long>(nrhs, cap);
 }
@@ -822,8 +885,6 @@ template <typename R>
 void Engine<R>::reserve_batch(int nrhs) {
   if (!batchable() || nrhs < 2) return;
   const int k = batch_chunk(nrhs);
-  long tot = 1;
-  for (int t = 0; t < d; t++) tot *= geom.E[t];
   if ((long)k * n_total > bgrid_cap) {
     NFFT_HIP_CHECK(R, hipStreamSynchronize(stream));
     hipFree(bgrid);
@@ -831,12 +892,12 @@ void Engine<R>::reserve_batch(int nrhs) {
     NFFT_HIP_CHECK(R, hipMalloc(&bgrid, sizeof(cplx<R>) * (size_t)k * n_total));
     bgrid_cap = (long)k * n_total;
   }
-  if ((long)k * sp_nsub * tot > btiles_cap) {
+  if ((long)k * tile_cells > btiles_cap) {
     NFFT_HIP_CHECK(R, hipStreamSynchronize(stream));
     hipFree(btiles);
     btiles = nullptr;
-    NFFT_HIP_CHECK(R, hipMalloc(&btiles, sizeof(cplx<R>) * (size_t)k * sp_nsub * tot));
-    btiles_cap = (long)k * sp_nsub * tot;
+    NFFT_HIP_CHECK(R, hipMalloc(&btiles, sizeof(cplx<R>) * (size_t)k * tile_cells));
+    btiles_cap = (long)k * tile_cells;
   }
 }
 
@@ -874,16 +935,14 @@ void Engine<R>::adjoint_batch(const cplx<R> *f_dev, cplx<R> *fhat_dev, int nrhs)
 }
 
 // batched adjoint in chunks of k right-hand sides on caller-given batch
-// grids (k n_total values) and tiles (k sp_nsub E^d values)
+// grids (k n_total values) and tiles (k tile_cells values)
 template <typename R>
 void Engine<R>::adjoint_batch_chunks(const cplx<R> *f_dev, cplx<R> *fhat_dev, int nrhs, int k,
                                      cplx<R> *grids, cplx<R> *tls) {
-  long tot = 1;
-  for (int t = 0; t < d; t++) tot *= geom.E[t];
   BinGeom gb = geom;
   gb.bs_g = n_total;
   gb.bs_f = M;
-  gb.bs_t = sp_nsub * tot;
+  gb.bs_t = tile_cells;
   for (int r0 = 0; r0 < nrhs; r0 += k) {
     const int nb = std::min(k, nrhs - r0);
     launch_spread<R>(f_dev + (long)r0 * M, grids, *this, stream, nb, &gb, tls);
@@ -898,22 +957,40 @@ void Engine<R>::adjoint_batch_chunks(const cplx<R> *f_dev, cplx<R> *fhat_dev, in
 // its grid and its spreading tiles, each rounded up to 256 bytes.
 template <typename R>
 long Engine<R>::noalloc_bytes_per_rhs() const {
-  long tot = 1;
-  for (int t = 0; t < d; t++) tot *= geom.E[t];
   auto up = [](long b) { return (b + 255) / 256 * 256; };
-  return up(n_total * (long)sizeof(cplx<R>)) + up(sp_nsub * tot * (long)sizeof(cplx<R>));
+  return up(n_total * (long)sizeof(cplx<R>)) + up(tile_cells * (long)sizeof(cplx<R>));
+}
+
+// What the entry point's limit is checked against: the bytes of the LDS-tile
+// kernels' batched adjoint, also for plans on the matrix-core kernels, so
+// that the plans it takes do not depend on the kernels (0: no limit, plans
+// those kernels run one right-hand side at a time).
+template <typename R>
+long Engine<R>::noalloc_limit_bytes() const {
+  if (!geom.mx) return noalloc_bytes_per_rhs();
+  if (!tile_batchable) return 0;
+  long tot = 1;
+  for (int t = 0; t < d; t++) tot *= tile_geom.E[t];
+  auto up = [](long b) { return (b + 255) / 256 * 256; };
+  return up(n_total * (long)sizeof(cplx<R>)) + up(tile_items * tot * (long)sizeof(cplx<R>));
 }
 
 template <typename R>
 int Engine<R>::adjoint_batch_noalloc(const cplx<R> *f_dev, cplx<R> *fhat_dev, int nrhs) {
-  if (nrhs < 2 || !batchable()) {
+  const long per = noalloc_bytes_per_rhs();
+  bool chunks = nrhs >= 2 && batchable();
+  if (chunks) {
+    const long limit = noalloc_limit_bytes();
+    if (limit > 0 && !noalloc_scratch) return -3;
+    if (limit > (long)kNoAllocScratchBytes) return -4;
+    // (a matrix-core plan's tiles may be larger than the limit's)
+    chunks = noalloc_scratch && per <= (long)kNoAllocScratchBytes;
+  }
+  if (!chunks) {
     // one by one on the plan's own grid and tiles
     for (int r = 0; r < nrhs; r++) adjoint(f_dev + (long)r * M, fhat_dev + (long)r * N_total);
     return 0;
   }
-  if (!noalloc_scratch) return -3;
-  const long per = noalloc_bytes_per_rhs();
-  if (per > (long)kNoAllocScratchBytes) return -4;
   const int k = (int)std::min<long>(nrhs, (long)kNoAllocScratchBytes / per);
   // k grids, then k tile sets, each block 256-byte aligned
   char *base = static_cast<char *>(noalloc_scratch);
@@ -958,7 +1035,10 @@ void Engine<R>::autotune() {
   // bin edges: the default, and the largest edge halved; in 1-D and 2-D also
   // every edge doubled and every edge halved; all within the LDS budget of
   // the default, nodes rebuilt for each, B and B^T timed together
-  if (!std::getenv("NFFT_HIP_BINS") && d <= 3) {
+  // (matrix-core plans have one kernel and one bin shape per window: only
+  // their FFT lines are timed)
+  const bool tune_b = !geom.mx;
+  if (tune_b && !std::getenv("NFFT_HIP_BINS") && d <= 3) {
     auto edges = [&]() {
       std::array<int, kMaxDim> e{};
       for (int t = 0; t < kMaxDim; t++) e[t] = geom.bs[t];
@@ -1011,7 +1091,7 @@ void Engine<R>::autotune() {
       build_nodes();
     }
   }
-  if (!std::getenv("NFFT_HIP_SPREAD")) {
+  if (tune_b && !std::getenv("NFFT_HIP_SPREAD")) {
     // float candidates accumulate in plain FP32 (the fixed-point LDS
     // variants are left out); double ones use ds_add_f64
     std::vector<int> cand;
@@ -1034,7 +1114,7 @@ void Engine<R>::autotune() {
   // spreading work-item size (nodes per item): half and twice the default,
   // the work lists rebuilt for each (fewer, longer items write fewer tiles
   // to reduce; more, shorter ones balance dense regions better)
-  if (!std::getenv("NFFT_HIP_SPREAD_ITEM") && d >= 2 && tile_scratch && sp_nsub > 0) {
+  if (tune_b && !std::getenv("NFFT_HIP_SPREAD_ITEM") && d >= 2 && tile_scratch && sp_nsub > 0) {
     const int base = spread_max_per_sub;
     float best = time_of([&]() { spread_to_grid(f); });
     int pick = base;
@@ -1053,7 +1133,7 @@ void Engine<R>::autotune() {
       build_nodes();
     }
   }
-  if (!std::getenv("NFFT_HIP_INTERP") && d >= 2) {
+  if (tune_b && !std::getenv("NFFT_HIP_INTERP") && d >= 2) {
     float best = 1e30f;
     int pick = interp_variant;
     for (int v : {0, 1}) {
@@ -1596,7 +1676,7 @@ struct PlanApi {
     if (rc)
       std::fprintf(stderr, "%sadjoint_batch_device_noalloc: %s (per right-hand side %ld bytes)\n",
                    sizeof(R) == 4 ? "nfftf_" : "nfft_", why,
-                   e->direct_only ? 0L : e->noalloc_bytes_per_rhs());
+                   e->direct_only ? 0L : e->noalloc_limit_bytes());
     return rc;
   }
 

@@ -1561,6 +1561,10 @@ void (*gather_zones_kernel(int d, long core, int &parts))(const cplx<R> *, const
 template <typename R>
 void launch_gather_tiles(const Engine<R> &e, cplx<R> *g, hipStream_t s, int nb, const BinGeom *gb,
                          cplx<R> *tiles) {
+  if (e.geom.mx) {
+    launch_mx_gather<R>(e, g, s, nb, gb, tiles);
+    return;
+  }
   long nbins = 1;
   for (int t = 0; t < e.geom.d; t++) nbins *= e.geom.nb[t];
   if (nb > 1) {
@@ -1763,6 +1767,10 @@ template <typename R>
 void launch_interp(const cplx<R> *g, cplx<R> *f, const Engine<R> &e, hipStream_t s, int nb,
                    const BinGeom *gb) {
   if (e.nsub == 0) return;
+  if (e.geom.mx) {
+    launch_mx_interp<R>(g, f, e, s, nb, gb);
+    return;
+  }
   const BinGeom &gg = gb ? *gb : e.geom;
   size_t lds;
   int threads;
@@ -1776,6 +1784,10 @@ template <typename R>
 void launch_spread(const cplx<R> *f, cplx<R> *g, const Engine<R> &e, hipStream_t s, int nb,
                    const BinGeom *gb, cplx<R> *tiles) {
   if (e.sp_nsub == 0) return;
+  if (e.geom.mx) {
+    launch_mx_spread<R>(f, e, s, nb, gb, tiles);
+    return;
+  }
   const BinGeom &gg = gb ? *gb : e.geom;
   size_t lds;
   int threads;
@@ -1809,6 +1821,7 @@ bool batch_kernels(const Engine<R> &e) {
     return false;
   } else {
     const BinGeom &gg = e.geom;
+    if (gg.mx) return true;
     if (!(e.tile_scratch && gg.zoned && gg.m >= 1 && gg.m <= kMaxStaticM)) return false;
     if (tile_bytes<R>(gg) > kTileBudget || e.interp_variant != 0) return false;
     if (gg.d == 3)
