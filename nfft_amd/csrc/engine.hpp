@@ -130,10 +130,10 @@ enum FftIn { kFromGrid = 0, kFromGridBand = 1, kFromCoeffs = 2 };
 enum FftOut { kToGrid = 0, kToGridBand = 1, kToCoeffs = 2 };
 
 // LDS line stride (complex elements) of the FFT passes: odd, with one pad
-// element per 16 (fft.hip)
+// element per 16 (fft.hpp)
 __host__ __device__ inline int lds_line_stride(int n) { return n + (n >> 4) + 1; }
 
-// One pruned pass of the oversampled FFT along dimension t (fft.hip): the
+// One pruned pass of the oversampled FFT along dimension t (fft.hpp): the
 // lines are all combinations of the other dimensions' coordinates, each
 // either over the full grid or over the band only (dimensions whose band is
 // all that is nonzero, or all that is needed).
@@ -152,11 +152,11 @@ template <typename R> struct FftPass {
   const R *phi_ax;
   const R *phi_od[kMaxDim - 1];
   long nlines;
-  int lines_per_block;
+  int lines_per_block;  // set by the launch, with twiddle_in_lds
   int nstages;
   int radix[20];
   const cplx<R> *twiddle;
-  int twiddle_in_lds;  // copy the twiddle table to LDS (when it fits 64 KB)
+  int twiddle_in_lds;  // copy the twiddle table to LDS (where it fits)
   // batched launches (blockIdx.y = right-hand side): offsets of the grid and
   // of the coefficient vectors per right-hand side
   long bs_g, bs_c;
@@ -176,7 +176,7 @@ template <typename R> struct FftPass {
   int nsub;     // lines per line of the other coordinates: n1 or n2
   int nfull;    // n
   int fn1, fn2;
-  const cplx<R> *twiddle_full;  // exp(-2 pi i k / n), k < n
+  const cplx<R> *twiddle_full;  // exp(-2 pi i j1 k2 / n) at j1 + n1 k2
   // grid buffer the pass reads and the one it writes: 0 the plan's grid, 1
   // its second grid (four-step plans only)
   int src, dst;

@@ -17,8 +17,10 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <mutex>
+#include <numeric>
 
 #include "../../include/nfft3.h"
 #include "../../include/nfft3_hip.h"
@@ -148,19 +150,49 @@ static void fit_window_polys(int m, long double b, std::vector<R> &out) {
       out[first + w * (DEG + 1) + i] = (i % 2 ? -1 : 1) * out[first + (2 * m + 1 - w) * (DEG + 1) + i];
 }
 
-// factor n into FFT radices: 8, 4, 2, the small primes with unrolled
-// butterflies, then any other prime factor (a generic stage, O(n p) per
-// line); at most 20 stages
+// Stages of an FFT of length n (fft.hpp), two at least: for lengths of prime
+// factors up to 13 the fewest radices of 2 .. 13, 15, 16 (each stage more is
+// an LDS pass more), of these the ones with the smallest largest radix and
+// then the smallest sum, largest first.  A larger prime factor is a generic
+// stage (O(n p) per line), which reads and writes LDS only: copies (radix 1)
+// go before and after.  At most 20 stages.
 static bool fft_radices(long n, std::vector<int> &out) {
   out.clear();
-  while (n % 8 == 0 && n > 1) { out.push_back(8); n /= 8; }
-  while (n % 4 == 0 && n > 1) { out.push_back(4); n /= 4; }
-  while (n % 2 == 0 && n > 1) { out.push_back(2); n /= 2; }
-  for (int p : {3, 5, 7, 11, 13})
-    while (n % p == 0) { out.push_back(p); n /= p; }
-  for (long p = 17; p * p <= n; p += 2)
-    while (n % p == 0) { out.push_back((int)p); n /= p; }
-  if (n > 1) out.push_back((int)n);
+  long r = n;
+  for (int p : {2, 3, 5, 7, 11, 13})
+    while (r % p == 0) r /= p;
+  if (r > 1) {
+    out.push_back(1);
+    for (int p : {8, 4, 2, 3, 5, 7, 11, 13})
+      while (n % p == 0) { out.push_back(p); n /= p; }
+    for (long p = 17; p * p <= n; p += 2)
+      while (n % p == 0) { out.push_back((int)p); n /= p; }
+    if (n > 1) out.push_back((int)n);
+    out.push_back(1);
+    return out.size() <= 20;
+  }
+  std::vector<int> best, cur;
+  auto better = [&]() {
+    if (best.empty() || cur.size() != best.size()) return best.empty() || cur.size() < best.size();
+    if (cur[0] != best[0]) return cur[0] < best[0];
+    return std::accumulate(cur.begin(), cur.end(), 0) < std::accumulate(best.begin(), best.end(), 0);
+  };
+  std::function<void(long, int)> search = [&](long left, int top) {
+    if (left == 1) {
+      if (better()) best = cur;
+      return;
+    }
+    if (!best.empty() && cur.size() >= best.size()) return;
+    for (int p : {16, 15, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2})
+      if (p <= top && left % p == 0) {
+        cur.push_back(p);
+        search(left / p, p);
+        cur.pop_back();
+      }
+  };
+  if (n > 1) search(n, 16);
+  if (best.size() < 2) best.insert(best.begin(), 2 - best.size(), 1);
+  out = best;
   return out.size() <= 20;
 }
 
@@ -580,12 +612,13 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
   // length factors into the stage radices is one pass; a longer one is
   // split into two four-step halves n = n1 n2 (split[t] = n1), each fitting.
   const int cap = sizeof(R) == 4 ? 4096 : 2048;  // elements per workgroup
-  auto twiddle_table = [&](long len) {
-    std::vector<cplx<R>> tw(len);
-    for (long k = 0; k < len; k++) {
-      long double a = -2.0L * kPiL * (long double)k / (long double)len;
+  auto fill_twiddles = [](std::vector<cplx<R>> &tw) {
+    for (size_t k = 0; k < tw.size(); k++) {
+      long double a = -2.0L * kPiL * (long double)k / (long double)tw.size();
       tw[k] = cplx<R>{(R)cosl(a), (R)sinl(a)};
     }
+  };
+  auto upload_table = [&](const std::vector<cplx<R>> &tw) {
     cplx<R> *dev = nullptr;
     NFFT_HIP_CHECK(R, hipMalloc(&dev, sizeof(cplx<R>) * tw.size()));
     NFFT_HIP_CHECK(R, hipMemcpy(dev, tw.data(), sizeof(cplx<R>) * tw.size(), hipMemcpyHostToDevice));
@@ -598,7 +631,9 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
     fft_radices(len, rad);
     ax.nstages = (int)rad.size();
     for (size_t i = 0; i < rad.size(); i++) ax.radix[i] = rad[i];
-    ax.twiddle = twiddle_table(len);
+    std::vector<cplx<R>> tw(len);
+    fill_twiddles(tw);
+    ax.twiddle = upload_table(tw);
     return ax;
   };
   long split[kMaxDim] = {};
@@ -627,7 +662,15 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
     axes.back().len = (int)n[t];
     sub1[t] = make_axis(n[t] / best);  // first half: length n2
     sub2[t] = make_axis(best);         // second half: length n1
-    tw_full[t] = twiddle_table(n[t]);
+    {
+      // w_n^(j1 k2) at k2 n1 + j1, where the first half writes its result
+      const long n1 = best, n2 = n[t] / best;
+      std::vector<cplx<R>> w(n[t]), tr(n[t]);
+      fill_twiddles(w);
+      for (long k2 = 0; k2 < n2; k2++)
+        for (long j1 = 0; j1 < n1; j1++) tr[k2 * n1 + j1] = w[j1 * k2];
+      tw_full[t] = upload_table(tr);
+    }
     extra_twiddles.push_back(sub1[t].twiddle);
     extra_twiddles.push_back(sub2[t].twiddle);
     extra_twiddles.push_back(tw_full[t]);
@@ -682,14 +725,9 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
       p.nsub = 1;
       p.nfull = (int)n[t];
       p.fn1 = p.fn2 = 1;
-      // lines per workgroup that fit the LDS budget (the launch may use
-      // fewer, see launch_fft_pass)
-      p.lines_per_block = (int)std::max<long>(1, std::min<long>(256, cap / n[t]));
       p.nstages = ax.nstages;
       for (int i = 0; i < p.nstages; i++) p.radix[i] = ax.radix[i];
       p.twiddle = ax.twiddle;
-      const size_t line_bytes = sizeof(cplx<R>) * (size_t)p.lines_per_block * lds_line_stride(p.len);
-      p.twiddle_in_lds = line_bytes + sizeof(cplx<R>) * (size_t)p.len <= 64 * 1024 ? 1 : 0;
       return p;
     };
     // a four-step axis: its two halves in place of one pass.  The first
@@ -718,9 +756,6 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
         q.nstages = ax.nstages;
         for (int i = 0; i < q.nstages; i++) q.radix[i] = ax.radix[i];
         q.twiddle = ax.twiddle;
-        q.lines_per_block = (int)std::max<long>(1, std::min<long>(256, cap / q.len));
-        const size_t lb = sizeof(cplx<R>) * (size_t)q.lines_per_block * lds_line_stride(q.len);
-        q.twiddle_in_lds = lb + sizeof(cplx<R>) * (size_t)q.len <= 64 * 1024 ? 1 : 0;
       }
       a.out_mode = kToGrid;
       b.in_mode = kFromGrid;
