@@ -13,7 +13,7 @@
 //        dimension-0 cell along a whole column of bins, so a wavefront keeps
 //        a ring of W planes and writes a plane out when the nodes have passed
 //        it: no LDS tile, no read-modify-write, no atomics.
-//   B    C[e1][k] += sum_{i, e2} g_i[e1][e2] (psi0_k[i] psi2_k[e2])
+//   B    C[e1][k] += psi0_k[i] (sum_e2 g_i[e1][e2] psi2_k[e2])
 //        for 16 nodes k: four 16 x 16 x 4 products per plane and part, then
 //        f_k = sum_e1 psi1_k[e1] C[e1][k].  A wavefront walks down the column
 //        with the planes its nodes reach in registers.
@@ -25,131 +25,20 @@
 // 5.5 cycles each between FP32 products), so the kernels are built to issue
 // few of them per node.  Measured against the LDS-tile kernels (spread_impl.hpp,
 // spread_runs.hpp), m = 4, 256^3 grid:
-//   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.70 + 0.36 (reduction)
+//   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.80 + 0.36 (reduction)
 //   B^T, FP64, 2^21 uniform nodes     3.49 + 1.87 ms -> 0.75 + 0.60
 //   B,   FP64, 2^21 uniform nodes     7.03 ms -> 0.96
 //   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.53 (k_mx_interp3s)
+// FP32 sums are cut so that no product sums more than 128 nodes (B^T) or the 16
+// positions of one plane (B): single sums over an item or a window lost up to a
+// bit (kooshball adjoint 3.0e-7 against FP64, 2.1e-7 as it is and before).
 // FP64 on sparse nodes (6 per column and plane) is bound by its grid traffic:
 // 256 / 49 grid cells read or written per cell, 41 planes per 32.
 #pragma once
 
-#include "engine.hpp"
-#include "window.hpp"
+#include "mx_util.hpp"
 
 namespace nfft_hip {
-
-template <typename R> struct MxTypes;
-template <> struct MxTypes<float> {
-  using v4 = float __attribute__((ext_vector_type(4)));
-};
-template <> struct MxTypes<double> {
-  using v4 = double __attribute__((ext_vector_type(4)));
-};
-template <typename R> using mx4 = typename MxTypes<R>::v4;
-
-// c + a b for a 16 x 4 operand a (lane l holds row l & 15, column l >> 4), a
-// 4 x 16 operand b (lane l: row l >> 4, column l & 15) and a 16 x 16 result
-// (lane l, element r: column l & 15 and row mx_row<R>(l, r)).
-__device__ __forceinline__ mx4<float> mx_mul(float a, float b, mx4<float> c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ mx4<double> mx_mul(double a, double b, mx4<double> c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-template <typename R> __device__ __forceinline__ int mx_row(int q, int r) {
-  return sizeof(R) == 4 ? 4 * q + r : q + 4 * r;
-}
-
-// DPP move within 16-lane rows: lane I of the row
-template <int CTRL> __device__ __forceinline__ float mx_dpp(float x) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL> __device__ __forceinline__ double mx_dpp(double x) {
-  const long long u = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(u & 0xffffffffLL), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-template <int I, typename R> __device__ __forceinline__ R mx_bcast(R x) {
-  return mx_dpp<0x150 + I>(x);
-}
-// sum over the four lanes of a column (l & 15), in every lane
-__device__ __forceinline__ float mx_col_sum(float x) {
-  const int v = __float_as_int(x);
-  auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  x = __int_as_float(a[0]) + __int_as_float(a[1]);
-  const int w = __float_as_int(x);
-  auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
-  return __int_as_float(b[0]) + __int_as_float(b[1]);
-}
-__device__ __forceinline__ double mx_col_sum(double x) {
-  x += __shfl_xor(x, 32, 64);
-  return x + __shfl_xor(x, 16, 64);
-}
-
-// Window rows of a chunk of nodes in LDS: row (t, node) holds the node's
-// dimension-t window over the positions, kMxPitch elements apart (rows of 16
-// or more positions; 20 spreads the 4 x 16 operand reads over the banks).
-constexpr int kMxPitch = 20;
-// coefficients per polynomial in the LDS table of plans whose dimensions
-// differ in sigma
-template <typename R> constexpr int kMxCoef = (poly_deg_v<R> + 4) / 4 * 4;
-
-// One window row: taps at positions shift .. shift + W - 1, zeros at the other
-// positions of the row.  Tap pairs (w, W-1-w) come from one polynomial's even
-// and odd parts at tt = frac - 1/2; pc(w) gives tap w's coefficients.
-template <typename R, int W, typename Coef>
-__device__ __forceinline__ void mx_window_row(R *row, int shift, R tt, Coef pc) {
-  constexpr int PD = poly_deg_v<R>;
-  constexpr int KE = PD - (PD % 2);      // highest even power
-  constexpr int KO = PD - 1 + (PD % 2);  // highest odd power
-  constexpr int V = 16 / sizeof(R);
-  using vec = R __attribute__((ext_vector_type(V)));
-#pragma unroll
-  for (int z = 0; z < kMxPitch; z += V) *reinterpret_cast<vec *>(row + z) = vec(0);
-  const R t2 = tt * tt;
-  R *at = row + shift;
-#pragma unroll
-  for (int w = 0; w < W / 2; w++) {
-    const R *c = pc(w);
-    R e = c[KE];
-#pragma unroll
-    for (int k = KE - 2; k >= 0; k -= 2) e = fma(e, t2, c[k]);
-    R o = c[KO];
-#pragma unroll
-    for (int k = KO - 2; k >= 1; k -= 2) o = fma(o, t2, c[k]);
-    at[w] = fma(tt, o, e);
-    at[W - 1 - w] = fma(-tt, o, e);
-  }
-}
-
-// copies the window polynomials of D dimensions (lower half of the taps) to
-// LDS, kMxCoef apart
-template <typename R, int D, int W>
-__device__ __forceinline__ void mx_load_poly(R *spoly, const R *poly, int tid, int nthr) {
-  constexpr int C = poly_deg_v<R> + 1, H = W / 2;
-  for (int i = tid; i < D * H * C; i += nthr) {
-    const int k = i % C, w = (i / C) % H, t = i / (C * H);
-    spoly[(t * H + w) * kMxCoef<R> + k] = poly[(t * W + w) * C + k];
-  }
-}
-
-// v[r] = 0 in place, for a branch of the node loop: a plain assignment made the
-// compiler copy all accumulators at the loop's head
-template <typename V> __device__ __forceinline__ void mx_clear(V &v, int r) {
-  auto x = v[r];
-  if constexpr (sizeof(x) == 4) asm("v_mov_b32 %0, 0" : "+v"(x));
-  else asm("v_mov_b64 %0, 0" : "+v"(x));
-  v[r] = x;
-}
-
-// a[i] = p1 times lane i of every 16-lane row of p0
-template <typename R, int H, int I = 0>
-__device__ __forceinline__ void mx_weights(R (&a)[H], R p0, R p1) {
-  a[I] = mx_bcast<I>(p0) * p1;
-  if constexpr (I + 1 < H) mx_weights<R, H, I + 1>(a, p0, p1);
-}
 
 // B^T of one work item: a run of nodes of one column (dimension-1 and -2
 // bins), sorted by dimension-0 cell.  Two wavefronts per item, each
@@ -160,7 +49,7 @@ __device__ __forceinline__ void mx_weights(R (&a)[H], R p0, R p1) {
 // enter with value zero).  Output: the item's planes of 16 x 16 cells in
 // scratch, summed into the grid by k_mx_gather3.
 template <typename R, int W, bool SHARED>
-__global__ __launch_bounds__(128, sizeof(R) == 4 ? 4 : 2) void k_mx_spread3(
+__global__ __launch_bounds__(128, sizeof(R) == 4 ? (W <= 10 ? 4 : 3) : 2) void k_mx_spread3(
     const cplx<R> *__restrict__ fin, cplx<R> *__restrict__ tiles, const int *__restrict__ perm,
     const int *__restrict__ cell, const R *__restrict__ frac, const int4 *__restrict__ subs,
     const int4 *__restrict__ info, BinGeom gg, WinParams<R> wp) {
@@ -185,9 +74,15 @@ __global__ __launch_bounds__(128, sizeof(R) == 4 ? 4 : 2) void k_mx_spread3(
     mx_load_poly<R, 3, W>(spoly, wp.poly, threadIdx.x, 128);
     __syncthreads();
   }
-  mx4<R> acc[H][2];
+  // FP32: a product's sum runs over 4 chunks, the sums of these over the item
+  // (one sum over the thousands of nodes of a dense item would lose a bit)
+  constexpr bool TWO = sizeof(R) == 4;
+  mx4<R> acc[H][2], sum[TWO ? H : 1][2];
 #pragma unroll
-  for (int i = 0; i < H; i++) acc[i][0] = acc[i][1] = mx4<R>{0, 0, 0, 0};
+  for (int i = 0; i < H; i++) {
+    acc[i][0] = acc[i][1] = mx4<R>{0, 0, 0, 0};
+    if constexpr (TWO) sum[i][0] = sum[i][1] = mx4<R>{0, 0, 0, 0};
+  }
   const int *cellp = cell + t * gg.M + sp.y;
   const R *fracp = frac + t * gg.M + sp.y;
   const int *permp = perm + sp.y;
@@ -223,6 +118,12 @@ __global__ __launch_bounds__(128, sizeof(R) == 4 ? 4 : 2) void k_mx_spread3(
           // (re, im) pairs across the node loop and moves all of them around
           // every product, 40 moves per 20 of them)
           R vr = acc[s][0][r], vi = acc[s][1][r];
+          if constexpr (TWO) {
+            vr += sum[s][0][r];
+            vi += sum[s][1][r];
+            mx_clear(sum[s][0], r);
+            mx_clear(sum[s][1], r);
+          }
           asm("" : "+v"(vr));
           asm("" : "+v"(vi));
           out[mx_row<R>(q, r) * 16] = cplx<R>{vr, vi};
@@ -283,6 +184,19 @@ __global__ __launch_bounds__(128, sizeof(R) == 4 ? 4 : 2) void k_mx_spread3(
       for (; k + 4 <= end; k += 4) four(k + q, true);
       if (k < end) four(min(k + q, NC - 1), k + q < end);
       k = end;
+    }
+    if constexpr (TWO) {
+      if ((base / NC) % 4 == 3) {
+#pragma unroll
+        for (int s = 0; s < H; s++)
+#pragma unroll
+          for (int x = 0; x < 2; x++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              sum[s][x][r] += acc[s][x][r];
+              mx_clear(acc[s][x], r);
+            }
+      }
     }
     __syncthreads();
   }
@@ -422,13 +336,15 @@ __global__ __launch_bounds__(64 * kMxParts<R>, sizeof(R) == 4 && W <= 10 ? 3 : 2
           const int p = ra + (s < rot ? s - rot + RW : s - rot);
           if (p >= ak && p < az + W) {
             const R w = w0[p];
-            R a[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) a[u] = w * a2[u];
+            mx4<R> z[NP] = {};
 #pragma unroll
             for (int u = 0; u < 4; u++)
 #pragma unroll
-              for (int x = 0; x < NP; x++) acc[x] = mx_mul(ring[s][x][u], a[u], acc[x]);
+              for (int x = 0; x < NP; x++) z[x] = mx_mul(ring[s][x][u], a2[u], z[x]);
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+              for (int x = 0; x < NP; x++) acc[x][u] = fma(w, z[x][u], acc[x][u]);
           }
         }
         // rows e1, columns nodes: four rows in the lane, 16 over its column
