@@ -201,35 +201,37 @@ __device__ __forceinline__ void node_window(const int *__restrict__ cell,
   }
 }
 
-// FP32 window of a node when every dimension shares one mirror-symmetric
+// Window of a node when every dimension shares one mirror-symmetric
 // tap table (wp.poly_shared): taps w and W-1-w come from the even part E and
 // odd part O of tap w's polynomial, psi = E(t^2) +- t O(t^2).  The W/2
 // polynomials of dimension 0 (W/2 * kPolyCoef values) stay in scalar
-// registers for the whole kernel instead of the d * W per-tap sets, and a
-// tap pair costs kPolyDeg + 1 FMAs instead of 2 kPolyDeg.
-template <int D, int W>
+// registers for the whole kernel (FP32) instead of the d * W per-tap sets, and
+// a tap pair costs one degree + 1 FMAs instead of two degrees (2-D FP64, m = 6,
+// 2^20 nodes: B 133 -> 97 us).
+template <typename R, int D, int W>
 __device__ __forceinline__ void node_window_sym(const int *__restrict__ cell,
-                                                const float *__restrict__ frac, long p, long M,
-                                                const WinParams<float> &wp, int (&c)[D],
-                                                float (&psi)[D][W]) {
-  constexpr int KE = kPolyDeg - (kPolyDeg % 2);  // highest even power
-  constexpr int KO = kPolyDeg - 1 + (kPolyDeg % 2);  // highest odd power
+                                                const R *__restrict__ frac, long p, long M,
+                                                const WinParams<R> &wp, int (&c)[D],
+                                                R (&psi)[D][W]) {
+  constexpr int PD = poly_deg_v<R>;
+  constexpr int KE = PD - (PD % 2);  // highest even power
+  constexpr int KO = PD - 1 + (PD % 2);  // highest odd power
 #pragma unroll
   for (int t = 0; t < D; t++) {
     c[t] = cell[t * M + p];
-    const float tt = frac[t * M + p] - 0.5f;
-    const float t2 = tt * tt;
+    const R tt = frac[t * M + p] - R(0.5);
+    const R t2 = tt * tt;
 #pragma unroll
     for (int w = 0; w < W / 2; w++) {
-      const float *pc = wp.poly + w * kPolyCoef;
-      float e = pc[KE];
+      const R *pc = wp.poly + w * (PD + 1);
+      R e = pc[KE];
 #pragma unroll
-      for (int k = KE - 2; k >= 0; k -= 2) e = fmaf(e, t2, pc[k]);
-      float o = pc[KO];
+      for (int k = KE - 2; k >= 0; k -= 2) e = fma(e, t2, pc[k]);
+      R o = pc[KO];
 #pragma unroll
-      for (int k = KO - 2; k >= 1; k -= 2) o = fmaf(o, t2, pc[k]);
-      psi[t][w] = fmaf(tt, o, e);
-      psi[t][W - 1 - w] = fmaf(-tt, o, e);
+      for (int k = KO - 2; k >= 1; k -= 2) o = fma(o, t2, pc[k]);
+      psi[t][w] = fma(tt, o, e);
+      psi[t][W - 1 - w] = fma(-tt, o, e);
     }
   }
 }
@@ -462,8 +464,8 @@ __global__ __launch_bounds__(256) void k_interp_tile(const cplx<R> *__restrict__
       int c[D], cb[D];
       R pa_[D][W], pb_[D][W];
       if constexpr (SYM) {
-        node_window_sym<D, W>(cell, frac, pa, gg.M, wp, c, pa_);
-        node_window_sym<D, W>(cell, frac, pb, gg.M, wp, cb, pb_);
+        node_window_sym<R, D, W>(cell, frac, pa, gg.M, wp, c, pa_);
+        node_window_sym<R, D, W>(cell, frac, pb, gg.M, wp, cb, pb_);
       } else {
         node_window<R, D, W>(cell, frac, pa, gg.M, wp, c, pa_);
         node_window<R, D, W>(cell, frac, pb, gg.M, wp, cb, pb_);
@@ -532,7 +534,7 @@ __global__ __launch_bounds__(256) void k_interp_tile(const cplx<R> *__restrict__
     const long p = (long)sp.y + i;
     int c[D];
     R psi[D][W];
-    if constexpr (SYM) node_window_sym<D, W>(cell, frac, p, gg.M, wp, c, psi);
+    if constexpr (SYM) node_window_sym<R, D, W>(cell, frac, p, gg.M, wp, c, psi);
     else node_window<R, D, W>(cell, frac, p, gg.M, wp, c, psi);
     R ar = 0, ai = 0;
     if constexpr (D == 1) {
@@ -1603,7 +1605,7 @@ template <typename R> struct BKernelTable {
   using fn = void (*)(const cplx<R> *, cplx<R> *, const int *, const int *, const R *,
                       const int4 *, BinGeom, WinParams<R>, cplx<R> *);
   fn interp_static[kMaxDim][kMaxStaticM + 1];
-  fn interp_sym[kMaxDim][kMaxStaticM + 1];   // float only, shared tap table
+  fn interp_sym[kMaxDim][kMaxStaticM + 1];   // shared tap table (double: d = 1, 2)
   fn interp_pair[kMaxDim][kMaxStaticM + 1];  // float d = 2, 3: node pairs of one cell
   fn interp_pair_sym[kMaxDim][kMaxStaticM + 1];
   fn spread_static[kMaxDim][kMaxStaticM + 1];
@@ -1629,7 +1631,8 @@ template <typename R> struct BKernelTable {
 template <typename R, int D, int M_>
 void bk_fill_one(BKernelTable<R> &k) {
   k.interp_static[D - 1][M_] = k_interp_tile<R, D, 2 * M_ + 2>;
-  if constexpr (std::is_same_v<R, float>) k.interp_sym[D - 1][M_] = k_interp_tile<R, D, 2 * M_ + 2, true>;
+  if constexpr (std::is_same_v<R, float> || D <= 2)
+    k.interp_sym[D - 1][M_] = k_interp_tile<R, D, 2 * M_ + 2, true>;
   if constexpr (std::is_same_v<R, float> && (D == 2 || D == 3)) {
     k.interp_pair[D - 1][M_] = k_interp_tile<R, D, 2 * M_ + 2, false, true>;
     k.interp_pair_sym[D - 1][M_] = k_interp_tile<R, D, 2 * M_ + 2, true, true>;
