@@ -1396,11 +1396,9 @@ __global__ __launch_bounds__(256) void k_gather_tiles(const cplx<R> *__restrict_
 // [bs-m, bs)); every work item of each of the 3^d neighbour bins contributes
 // one contiguous zone.  The (zone, work item) pairs are listed in LDS; each
 // thread owns CPT core cells, sums in registers and keeps up to 16 loads in
-// flight; each grid cell is written once.  P workgroups share a bin, each
-// summing CPT * 256 of its core cells, so the heavy neighbourhoods of dense
-// regions (hundreds of contributions) are spread over P workgroups.
+// flight; each grid cell is written once.
 constexpr int kZonePairs = 512;  // pairs listed per pass
-template <typename R, int D, int CPT, int P = 1>
+template <typename R, int D, int CPT>
 __global__ __launch_bounds__(256) void k_gather_zones(const cplx<R> *__restrict__ tiles,
                                                       const int *__restrict__ sp_first,
                                                       const int *__restrict__ sp_count,
@@ -1418,7 +1416,7 @@ __global__ __launch_bounds__(256) void k_gather_zones(const cplx<R> *__restrict_
   __shared__ int s_pz[kZonePairs];
   int bc[3] = {0, 0, 0};
   {
-    int r = order[blockIdx.x / P];  // heavy neighbourhoods first
+    int r = order[blockIdx.x];  // heavy neighbourhoods first
 #pragma unroll
     for (int t = D - 1; t >= 0; t--) {
       bc[t] = r % gg.nb[t];
@@ -1469,13 +1467,11 @@ __global__ __launch_bounds__(256) void k_gather_zones(const cplx<R> *__restrict_
   int core = 1;
 #pragma unroll
   for (int t = 0; t < D; t++) core *= gg.bs[t];
-  // this workgroup's slice of the core cells
-  const int qbase = (int)(blockIdx.x % P) * CPT * (int)blockDim.x;
   int kc[CPT][3];
   R ar[CPT], ai[CPT];
 #pragma unroll
   for (int i = 0; i < CPT; i++) {
-    const int q = qbase + threadIdx.x + i * blockDim.x;
+    const int q = threadIdx.x + i * blockDim.x;
     int rem = q < core ? q : 0;
     kc[i][0] = kc[i][1] = kc[i][2] = 0;
 #pragma unroll
@@ -1504,7 +1500,7 @@ __global__ __launch_bounds__(256) void k_gather_zones(const cplx<R> *__restrict_
         const long pb = i < nw ? s_pbase[i] : 0;
 #pragma unroll
         for (int c = 0; c < CPT; c++) {
-          const int q = qbase + threadIdx.x + c * blockDim.x;
+          const int q = threadIdx.x + c * blockDim.x;
           bool in = i < nw && q < core;
           int idx = 0;
 #pragma unroll
@@ -1528,7 +1524,7 @@ __global__ __launch_bounds__(256) void k_gather_zones(const cplx<R> *__restrict_
   }
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
-    const int q = qbase + threadIdx.x + c * blockDim.x;
+    const int q = threadIdx.x + c * blockDim.x;
     if (q >= core) break;
     long gi = 0;
 #pragma unroll
@@ -1537,27 +1533,91 @@ __global__ __launch_bounds__(256) void k_gather_zones(const cplx<R> *__restrict_
   }
 }
 
-// zone reduction for d dimensions and core cells per bin; parts: workgroups
-// per bin (parts x CPT x 256 >= core)
-template <typename R>
-void (*gather_zones_kernel(int d, long core, int &parts))(const cplx<R> *, const int *, const int *,
-                                                         cplx<R> *, BinGeom, const int *) {
-  parts = 1;
-  // 3-D keeps one workgroup per bin (two measured slower on the kooshball:
-  // 0.25 -> 0.33 ms); 2-D splits 1024-cell cores four ways (clustered 512^2:
-  // 0.38 -> 0.32 ms per trafo + adjoint)
-  if (d == 3)
-    return core <= 512 ? k_gather_zones<R, 3, 2>
-                       : (core <= 1024 ? k_gather_zones<R, 3, 4> : k_gather_zones<R, 3, 16>);
-  if (d == 2) {
-    if (core <= 256) return k_gather_zones<R, 2, 1>;
-    if (core <= 1024) {
-      parts = 4;
-      return k_gather_zones<R, 2, 1, 4>;
-    }
-    return k_gather_zones<R, 2, 16>;
+// The same reduction for d = 1, 2: a thread owns one core cell and knows its
+// place in each of the 3^d zones, so that the loop over the items has no lists
+// or tables in LDS, and up to U items of all neighbours are in flight at once.
+// `parts` workgroups share a bin.  Bound: the chain order -> first item -> tile
+// values -> grid cell, and in dense regions a load more per U items of a bin.
+// 512^2 grid, 128512 radial nodes in 987 items, some 60 in the heaviest
+// neighbourhood: 17 us with k_gather_zones, 9 here.
+template <typename R, int D>
+__global__ __launch_bounds__(256) void k_gather_zones_cell(const cplx<R> *__restrict__ tiles,
+                                                           const int *__restrict__ sp_first,
+                                                           const int *__restrict__ sp_count,
+                                                           cplx<R> *__restrict__ g, BinGeom gg,
+                                                           const int *__restrict__ order,
+                                                           int parts) {
+  static_assert(D == 1 || D == 2, "3-D: k_gather_zones");
+  constexpr int NZ = D == 1 ? 3 : 9, U = 2;
+  // right-hand side blockIdx.y of a batched launch
+  tiles += (long)blockIdx.y * gg.bs_t;
+  g += (long)blockIdx.y * gg.bs_g;
+  const int bin = order[blockIdx.x / parts];  // heavy neighbourhoods first
+  // (1-D: as a second dimension of one bin and cell)
+  const int nb1 = D == 2 ? gg.nb[1] : 1, bs1 = D == 2 ? gg.bs[1] : 1;
+  const int b0 = bin / nb1, b1 = bin - b0 * nb1;
+  const long tot = (long)gg.E[0] * (D == 2 ? gg.E[1] : 1);
+  const int core = gg.bs[0] * bs1;
+  const int q = (int)(blockIdx.x % parts) * 256 + threadIdx.x;
+  const int k0 = q / bs1, k1 = q - k0 * bs1;
+  const cplx<R> *tp[NZ];
+  int cnt[NZ], most = 0;
+#pragma unroll
+  for (int z = 0; z < NZ; z++) {
+    int v0 = b0 + (D == 2 ? z / 3 : z) - 1, v1 = D == 2 ? b1 + z % 3 - 1 : 0;
+    v0 += v0 < 0 ? gg.nb[0] : (v0 >= gg.nb[0] ? -gg.nb[0] : 0);
+    v1 += v1 < 0 ? nb1 : (v1 >= nb1 ? -nb1 : 0);
+    const int nbl = v0 * nb1 + v1, n = sp_count[nbl];
+    const int *zd = gg.zdesc + 8 * z;  // its zone's place in the tile and in this core
+    const int u0 = k0 - zd[1], u1 = D == 2 ? k1 - zd[2] : 0;
+    const bool in = q < core && u0 >= 0 && u0 < zd[4] && (D == 1 || (u1 >= 0 && u1 < zd[5]));
+    cnt[z] = in ? n : 0;
+    most = max(most, n);
+    tp[z] = tiles + (long)sp_first[nbl] * tot + zd[0] + (D == 2 ? u0 * zd[5] + u1 : u0);
   }
-  return core <= 1024 ? k_gather_zones<R, 1, 4> : k_gather_zones<R, 1, 16>;
+  R ar = 0, ai = 0;
+  for (int c = 0; c < most; c += U) {
+    cplx<R> v[U][NZ];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int z = 0; z < NZ; z++) {
+        v[u][z] = cplx<R>{0, 0};
+        if (c + u < cnt[z]) v[u][z] = tp[z][(long)(c + u) * tot];
+      }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int z = 0; z < NZ; z++) {
+        ar += v[u][z].x;
+        ai += v[u][z].y;
+      }
+  }
+  if (q < core)
+    g[(long)(b0 * gg.bs[0] + k0) * (D == 2 ? gg.n[1] : 1) + b1 * bs1 + k1] = cplx<R>{ar, ai};
+}
+
+// zone reduction of nb right-hand sides
+template <typename R>
+void launch_gather_zones(const cplx<R> *tiles, const Engine<R> &e, cplx<R> *g, const BinGeom &gg,
+                         hipStream_t s, int nb) {
+  long core = 1, nbins = 1;
+  for (int t = 0; t < gg.d; t++) {
+    core *= gg.bs[t];
+    nbins *= gg.nb[t];
+  }
+  if (gg.d <= 2) {
+    const int parts = (int)((core + 255) / 256);
+    auto fn = gg.d == 1 ? k_gather_zones_cell<R, 1> : k_gather_zones_cell<R, 2>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)(nbins * parts), (unsigned)nb), dim3(256), 0, s, tiles,
+                       e.sp_first, e.sp_count, g, gg, e.bin_order, parts);
+    return;
+  }
+  // one workgroup per bin (two measured slower on the kooshball: 0.25 -> 0.33 ms)
+  auto fn = core <= 512 ? k_gather_zones<R, 3, 2>
+                        : (core <= 1024 ? k_gather_zones<R, 3, 4> : k_gather_zones<R, 3, 16>);
+  hipLaunchKernelGGL(fn, dim3((unsigned)nbins, (unsigned)nb), dim3(256), 0, s, tiles, e.sp_first,
+                     e.sp_count, g, gg, e.bin_order);
 }
 
 template <typename R>
@@ -1569,30 +1629,10 @@ void launch_gather_tiles(const Engine<R> &e, cplx<R> *g, hipStream_t s, int nb, 
   }
   long nbins = 1;
   for (int t = 0; t < e.geom.d; t++) nbins *= e.geom.nb[t];
-  if (nb > 1) {
-    // batched: the zone reduction reads the right-hand side from blockIdx.y
-    using F = void (*)(const cplx<R> *, const int *, const int *, cplx<R> *, BinGeom, const int *);
-    long core = 1;
-    for (int t = 0; t < e.geom.d; t++) core *= e.geom.bs[t];
-    int parts = 1;
-    F fz = gather_zones_kernel<R>(e.geom.d, core, parts);
-    hipLaunchKernelGGL(fz, dim3((unsigned)(nbins * parts), (unsigned)nb), dim3(256), 0, s, tiles,
-                       e.sp_first,
-                       e.sp_count, g, *gb, e.bin_order);
+  // (only zoned plans run batches in one launch)
+  if (nb > 1 || e.geom.zoned) {
+    launch_gather_zones<R>(nb > 1 ? tiles : e.tiles, e, g, nb > 1 ? *gb : e.geom, s, nb);
     return;
-  }
-  if (e.geom.zoned) {
-    long core = 1;
-    for (int t = 0; t < e.geom.d; t++) core *= e.geom.bs[t];
-    if (core <= 4096) {
-      using F = void (*)(const cplx<R> *, const int *, const int *, cplx<R> *, BinGeom,
-                         const int *);
-      int parts = 1;
-      F fz = gather_zones_kernel<R>(e.geom.d, core, parts);
-      hipLaunchKernelGGL(fz, dim3((unsigned)(nbins * parts)), dim3(256), 0, s, e.tiles, e.sp_first,
-                         e.sp_count, g, e.geom, e.bin_order);
-      return;
-    }
   }
   auto fn = e.geom.d == 1 ? k_gather_tiles<R, 1> : e.geom.d == 2 ? k_gather_tiles<R, 2>
                                                                  : k_gather_tiles<R, 3>;
