@@ -280,6 +280,26 @@ __global__ void k_fill_subs(const int *__restrict__ hist, const int *__restrict_
 // count), so that the few long-running workgroups of dense regions start at
 // the beginning of the launch instead of ending it.
 constexpr int kOrderBuckets = 16;
+
+// atomicAdd(&count[bucket], 1) for every active lane, one atomic per bucket
+// and wavefront (16384 lanes on a few counters one by one took 187 us)
+__device__ __forceinline__ int bucket_add(int *count, int bucket) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long left = __ballot(1);
+  int at = 0;
+  while (left) {
+    const int lead = __builtin_ctzll(left);
+    const int b = __shfl(bucket, lead, 64);
+    const unsigned long long same = __ballot(bucket == b) & left;
+    int first = 0;
+    if (lane == lead) first = atomicAdd(&count[b], __popcll(same));
+    first = __shfl(first, lead, 64);
+    if (bucket == b) at = first + __popcll(same & ((1ull << lane) - 1));
+    left &= ~same;
+  }
+  return at;
+}
+
 __global__ void k_bin_weight(const int *__restrict__ count_of, BinGeom gg, long nbins,
                              int *__restrict__ bucket_of, int *__restrict__ bucket_hist) {
   long b = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -312,14 +332,14 @@ __global__ void k_bin_weight(const int *__restrict__ count_of, BinGeom gg, long 
   while (lg < kOrderBuckets - 1 && (2l << lg) <= pairs + 1) lg++;
   const int bucket = kOrderBuckets - 1 - lg;  // heaviest first
   bucket_of[b] = bucket;
-  atomicAdd(&bucket_hist[bucket], 1);
+  bucket_add(bucket_hist, bucket);
 }
 
 __global__ void k_bin_order(const int *__restrict__ bucket_of, long nbins,
                             int *__restrict__ bucket_next, int *__restrict__ order) {
   long b = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nbins) return;
-  order[atomicAdd(&bucket_next[bucket_of[b]], 1)] = (int)b;
+  order[bucket_add(bucket_next, bucket_of[b])] = (int)b;
 }
 
 // Launch order of the work items: largest node counts first (buckets by
@@ -333,14 +353,14 @@ __global__ void k_sub_weight(const int4 *__restrict__ subs, long nsub, int *__re
   while (lg < kOrderBuckets - 1 && (2 << lg) <= c) lg++;
   const int bucket = kOrderBuckets - 1 - lg;
   bucket_of[i] = bucket;
-  atomicAdd(&bucket_hist[bucket], 1);
+  bucket_add(bucket_hist, bucket);
 }
 
 __global__ void k_sub_order(const int4 *__restrict__ in, const int *__restrict__ bucket_of,
                             long nsub, int *__restrict__ bucket_next, int4 *__restrict__ out) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nsub) return;
-  out[atomicAdd(&bucket_next[bucket_of[i]], 1)] = in[i];
+  out[bucket_add(bucket_next, bucket_of[i])] = in[i];
 }
 
 // Interpolation slots: up to Q consecutive nodes of one cell run (same
