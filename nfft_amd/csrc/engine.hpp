@@ -74,12 +74,23 @@ struct BinGeom {
   int mx_span[3];
 };
 
+// the library's static scratch for allocation-free batched adjoints (plan.hip)
+constexpr long kNoAllocScratchBytes = 64L << 20;
+
 // Ragged bins: first cell of bin b of nb over n cells, and the bin of cell c
 // (n <= kMxMaxN, so that the products fit an int)
 constexpr int kMxMaxN = 32767;
 __host__ __device__ inline int mx_lo(int b, int n, int nb) { return b * n / nb; }
 __host__ __device__ inline int mx_bin(int c, int n, int nb) { return ((c + 1) * nb - 1) / n; }
-// widest window of the matrix-core kernels: m = kMxMaxM
+// 2-D matrix-core B^T (spread_mx2d.hpp): widest tile and window, wavefronts per
+// item, right-hand sides per workgroup of a batch, nodes summed in FP32 before
+// the sums are summed
+constexpr int kMx2dMaxE = 48;
+constexpr int kMx2dMaxM = 8;
+template <typename R> constexpr int kMx2dWaves = sizeof(R) == 4 ? 4 : 2;
+constexpr int kMx2dRhs = 2;
+constexpr int kMx2dOneSum = 64;
+// widest window of the 3-D matrix-core kernels: m = kMxMaxM
 constexpr int kMxMaxM = 6;
 
 // Kaiser-Bessel window of one dimension, scaled by 1/phi(0) so that the B
@@ -242,7 +253,8 @@ template <typename R> struct Engine {
   int4 *mx_bin_info = nullptr;
   int *mx_multi = nullptr;
   long mx_bins_cap = 0, mx_multi_n = 0;
-  // the bins that the LDS-tile kernels would use for a matrix-core plan, and
+  // the bins that the LDS-tile kernels would use for a matrix-core plan (d = 0:
+  // no such plan), and
   // whether they would run its batches in one launch: the allocation-free
   // batched adjoint accepts the same plans whichever kernels run
   BinGeom tile_geom{};
@@ -281,7 +293,8 @@ template <typename R> struct Engine {
   // spreading also 2 private tile per wavefront (priv), 3 row-partitioned
   // tile (rows), the FP32 3-D run-merging kernels 10 (runs2sbc: two node
   // streams per wavefront) and 13 (runs2rs: one stream, runs load and store
-  // their tile cells), and the 2-D run-merging kernel 14 (runs2d).
+  // their tile cells), the 2-D run-merging kernel 14 (runs2d)
+  // and the 2-D matrix-core kernel 15 (mx2d).
   // Set at plan creation; NFFT_HIP_INTERP / NFFT_HIP_SPREAD = name override.
   int interp_variant = 0;
   int spread_variant = 1;
@@ -302,6 +315,7 @@ template <typename R> struct Engine {
   void create(int d_, const long *N_, const long *n_, long M_, int m_);
   void set_bins(const int *bs);
   void set_mx_bins();
+  void set_mx2d_bins();
   void destroy();
   void upload_nodes(const R *x_host);
   void build_nodes();  // from xdev

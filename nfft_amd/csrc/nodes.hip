@@ -525,7 +525,7 @@ void bin_nodes(Engine<R> &e) {
   const long b_tiles = al(std::max(ntiles, ceil_div(M + 1, kScanTile)) * (long)sizeof(int));
   // the bins of the LDS-tile kernels a matrix-core plan would otherwise use
   long ntbins = 0;
-  if (gg.mx && e.tile_batchable) {
+  if (e.tile_batchable) {
     ntbins = 1;
     for (int t = 0; t < gg.d; t++) ntbins *= e.tile_geom.nb[t];
   }
@@ -757,6 +757,25 @@ void bin_nodes(Engine<R> &e) {
     e.mx_multi_n = totals[1];
     e.tile_cells = (totals[0] + (long)totals[1] * (gg.bs[0] + 2 * gg.m + 1)) * 256L;
     e.tile_items = totals[2];
+  }
+  if (!gg.mx && ntbins > 0 && e.sp_nsub > 0) {
+    // the LDS-tile kernels' items in the bins they would use: counted where a
+    // bound on them does not settle the limit they serve
+    long tot = 1;
+    for (int t = 0; t < gg.d; t++) tot *= e.tile_geom.E[t];
+    e.tile_items = std::min(M, ntbins + M / e.tile_spread_max_per_sub);
+    if ((tot * e.tile_items + e.n_total) * (long)sizeof(cplx<R>) + 512 > kNoAllocScratchBytes) {
+      int items = 0;
+      launch_fill_zero_int(sums + 1, 1, s);
+      launch_fill_zero_int(hist, ntbins, s);
+      hipLaunchKernelGGL(k_tile_bin_hist, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s, e.cell,
+                         e.tile_geom, hist);
+      hipLaunchKernelGGL(k_tile_items, dim3(1), dim3(256), 0, s, hist, ntbins,
+                         e.tile_spread_max_per_sub, e.spread_max_items, sums + 1);
+      NFFT_HIP_CHECK(R, hipMemcpyAsync(&items, sums + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+      NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
+      e.tile_items = items;
+    }
   }
   // heavy bins first for the zone reduction (the interpolation list's
   // temporaries are free again: bucket per bin, bucket histogram and offsets)

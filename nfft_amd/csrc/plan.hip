@@ -42,7 +42,6 @@ namespace nfft_hip {
 // stand-in for the symbol; its device address on each GPU comes from
 // hipGetSymbolAddress, looked up once per device when the first plan is
 // created there, and only that address is handed to kernels.
-constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
 constexpr int kNoAllocMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 static std::mutex g_scratch_mu;
@@ -466,6 +465,33 @@ void Engine<R>::set_mx_bins() {
   while (spread_max_per_sub > 512 && spread_max_per_sub * 2048L > M) spread_max_per_sub /= 2;
 }
 
+// Bin edges of 2-D plans on the matrix-core B^T in place of those set by
+// set_bins: the divisor of the grid length nearest to 16 for which the zone
+// reduction works (m + 1 cells or more) and the tile keeps two blocks of 16
+// cells (wider windows: three), or 16 where there is none.  Two blocks cost
+// half the products of three and the reduction fewer items per bin: 2^20
+// clustered nodes on 1024^2 with bins of 32 cells -> 16, m = 4 FP32: B^T 84 ->
+// 69 us, reduction 53 -> 22, B 34 -> 29; m = 6 FP64: 243 -> 155, 54 -> 24,
+// 114 -> 133.
+template <typename R>
+void Engine<R>::set_mx2d_bins() {
+  if (d != 2 || spread_variant != 15 || m < 1 || m > kMx2dMaxM) return;
+  const int W = 2 * m + 2;
+  int bs[kMaxDim];
+  for (int t = 0; t < kMaxDim; t++) bs[t] = 1;
+  for (int t = 0; t < d; t++) {
+    bs[t] = (int)std::min<long>(n[t], 16);
+    int best = 0;
+    for (int b = std::max(8, m + 1); b <= (W <= 16 ? 33 - W : 16); b++)
+      if (n[t] % b == 0 && (!best || std::abs(b - 16) <= std::abs(best - 16))) best = b;
+    if (best) bs[t] = best;
+  }
+  tile_geom = geom;
+  tile_batchable = batch_kernels<R>(*this);
+  tile_spread_max_per_sub = spread_max_per_sub;
+  set_bins(bs);
+}
+
 template <typename R>
 void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) {
   d = d_;
@@ -588,6 +614,7 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
     return std::strcmp(v, "runs2sbc") == 0  ? 10
            : std::strcmp(v, "runs2rs") == 0 ? 13
            : std::strcmp(v, "runs2d") == 0 ? 14
+           : std::strcmp(v, "mx2d") == 0 ? 15
            : std::strcmp(v, "rows") == 0 ? 3
            : std::strcmp(v, "priv") == 0 ? 2
            : std::strcmp(v, "wave") == 0 ? 1
@@ -599,13 +626,15 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
   if (const char *v = std::getenv("NFFT_HIP_PAIRS")) pair_interp = std::atoi(v) != 0;
   if (const char *v = std::getenv("NFFT_HIP_SLOT")) slot_nodes = std::atoi(v) >= 4 ? 4 : 2;
   if (const char *v = std::getenv("NFFT_HIP_SLOTSORT")) slot_sort = std::atoi(v) != 0;
-  // float: plain FP32 read-modify-write by wavefronts that own disjoint
-  // cells, same-cell runs summed in registers (3-D: two wavefronts per tile
-  // split by row parity; 2-D: one wavefront per tile; 1-D: private tiles);
-  // double: wavefronts sharing a tile with ds_add_f64
-  spread_variant = variant("NFFT_HIP_SPREAD", sizeof(R) == 4 ? (d == 3 ? 10 : (d == 2 ? 14 : 2)) : 1);
+  // 2-D: matrix cores (tiles wider than kMx2dMaxE cells and windows beyond
+  // kMx2dMaxM: as follows).  float: plain FP32 read-modify-write by wavefronts
+  // that own disjoint cells, same-cell runs summed in registers (3-D: two
+  // wavefronts per tile split by row parity; 2-D: one wavefront per tile; 1-D:
+  // private tiles); double: wavefronts sharing a tile with ds_add_f64
+  spread_variant = variant("NFFT_HIP_SPREAD", d == 2 ? 15 : (sizeof(R) == 4 ? (d == 3 ? 10 : 2) : 1));
 
   set_mx_bins();
+  if (!std::getenv("NFFT_HIP_BINS")) set_mx2d_bins();
 
   // FFT: twiddles per dimension, then the pruned passes of both directions.
   // An axis whose lines fit one workgroup's LDS (cap elements) and whose
@@ -997,12 +1026,12 @@ long Engine<R>::noalloc_bytes_per_rhs() const {
 }
 
 // What the entry point's limit is checked against: the bytes of the LDS-tile
-// kernels' batched adjoint, also for plans on the matrix-core kernels, so
+// kernels' batched adjoint, also for plans with matrix-core bins, so
 // that the plans it takes do not depend on the kernels (0: no limit, plans
 // those kernels run one right-hand side at a time).
 template <typename R>
 long Engine<R>::noalloc_limit_bytes() const {
-  if (!geom.mx) return noalloc_bytes_per_rhs();
+  if (tile_geom.d == 0) return noalloc_bytes_per_rhs();
   if (!tile_batchable) return 0;
   long tot = 1;
   for (int t = 0; t < d; t++) tot *= tile_geom.E[t];
@@ -1131,8 +1160,8 @@ void Engine<R>::autotune() {
     // variants are left out); double ones use ds_add_f64
     std::vector<int> cand;
     if (sizeof(R) == 4 && d == 3) cand = {10, 13, 3};
-    else if (sizeof(R) == 4 && d == 2) cand = {14, 1, 0, 2};
-    else if (sizeof(R) == 8 && d == 2) cand = {14, 1, 0};
+    else if (sizeof(R) == 4 && d == 2) cand = {15, 14, 1, 0, 2};
+    else if (sizeof(R) == 8 && d == 2) cand = {15, 14, 1, 0};
     else if (sizeof(R) == 8 && d >= 2) cand = {1, 0};
     float best = 1e30f;
     int pick = spread_variant;

@@ -1073,6 +1073,7 @@ __global__ __launch_bounds__(64 * NW) void k_spread_rows(const cplx<R> *__restri
 #include "spread_rows.hpp"
 #include "spread_runs.hpp"
 #include "spread_runs2d.hpp"
+#include "spread_mx2d.hpp"
 namespace nfft_hip {
 
 // ==================================================================== runtime m
@@ -1664,6 +1665,11 @@ template <typename R> struct BKernelTable {
   fn spread_runs2d[kMaxStaticM + 1];          // d = 2: run-merging, kRunWaves2d wavefronts
   fn spread_runs2d_1w[kMaxStaticM + 1];       // same, one wavefront (large tiles)
   fn spread_runs2d_mc[kMaxStaticM + 1];       // same, kRhsPerGroup right-hand sides each
+  // d = 2 on the matrix cores: [blocks per dimension - 2][window table shared]
+  // [sums of sums, float]; two blocks of single sums with kMx2dRhs right-hand
+  // sides per workgroup (float; the others would take over half the registers)
+  fn spread_mx2d[2][2][2][kMx2dMaxM + 1];
+  fn spread_mx2d_mc[2][kMx2dMaxM + 1];
   fn interp_rt[kMaxDim][2];  // [d-1][tile]
   fn spread_rt[kMaxDim][2];
 };
@@ -1684,6 +1690,21 @@ void bk_fill_one(BKernelTable<R> &k) {
     k.spread_priv[D - 1][M_] = k_spread_wave_priv<R, D, 2 * M_ + 2>;
   }
   if constexpr (D == 3 && D * (2 * M_ + 2) <= 64) k.spread_rows[M_] = k_spread_rows2<R, 2 * M_ + 2, 2>;
+  if constexpr (D == 2 && M_ <= kMx2dMaxM) {
+    constexpr bool TWO = std::is_same_v<R, float>;
+    k.spread_mx2d[0][0][0][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, 1, false, false>;
+    k.spread_mx2d[0][1][0][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, 1, true, false>;
+    k.spread_mx2d[1][0][0][M_] = k_spread_mx2d<R, 2 * M_ + 2, 3, 1, false, false>;
+    k.spread_mx2d[1][1][0][M_] = k_spread_mx2d<R, 2 * M_ + 2, 3, 1, true, false>;
+    k.spread_mx2d[0][0][1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, 1, false, TWO>;
+    k.spread_mx2d[0][1][1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, 1, true, TWO>;
+    k.spread_mx2d[1][0][1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 3, 1, false, TWO>;
+    k.spread_mx2d[1][1][1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 3, 1, true, TWO>;
+    if constexpr (std::is_same_v<R, float>) {
+      k.spread_mx2d_mc[0][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, kMx2dRhs, false, false>;
+      k.spread_mx2d_mc[1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, kMx2dRhs, true, false>;
+    }
+  }
   if constexpr (D == 2) {
     // FP64 factors take twice the registers: smaller node groups
     constexpr int G2 = std::is_same_v<R, float> ? ((2 * M_ + 2) * (M_ + 1) > 64 ? 4 : 8)
@@ -1746,12 +1767,20 @@ size_t tile_bytes(const BinGeom &gg) {
 // LDS tiles above this size use the global-memory variant
 constexpr size_t kTileBudget = 64 * 1024;
 
+// Blocks of 16 cells per dimension that the matrix-core 2-D B^T needs for a
+// plan's tiles (2 or 3), or 0 where it does not cover them
+inline int mx2d_blocks(const BinGeom &gg, int variant) {
+  if (variant != 15 || gg.d != 2 || gg.m < 1 || gg.m > kMx2dMaxM) return 0;
+  const int e = std::max(gg.E[0], gg.E[1]);
+  return e <= 32 ? 2 : (e <= kMx2dMaxE ? 3 : 0);
+}
+
 // variant: 0 lane per node, 1 wave per node, 2 wave per node with a private
 // tile (spreading only); falls back to what exists for (d, m)
 template <typename R>
 typename BKernelTable<R>::fn pick_bkernel(const BKernelTable<R> &k, const BinGeom &gg,
                                           bool spread, int variant, size_t &lds, int &threads,
-                                          bool shared_poly = false) {
+                                          bool shared_poly = false, bool two_sums = false) {
   size_t bytes = tile_bytes<R>(gg);
   // the lane-per-node 3-D interpolation tile has planes gg.ipp cells apart
   if (!spread && variant == 0 && gg.d == 3) bytes = (size_t)gg.E[0] * gg.ipp * sizeof(cplx<R>);
@@ -1760,6 +1789,15 @@ typename BKernelTable<R>::fn pick_bkernel(const BKernelTable<R> &k, const BinGeo
   threads = 256;
   if (tile && gg.d <= 3 && gg.m >= 1 && gg.m <= kMaxStaticM) {
     const int t = gg.d - 1;
+    if (spread && variant == 15 && gg.d == 2) {
+      if (const int blocks = mx2d_blocks(gg, variant)) {
+        threads = 64 * kMx2dWaves<R>;
+        lds = 0;
+        return k.spread_mx2d[blocks - 2][shared_poly ? 1 : 0][two_sums ? 1 : 0][gg.m];
+      }
+      // wider tiles
+      variant = sizeof(R) == 4 ? 14 : 1;
+    }
     if (spread && variant == 14 && gg.d == 2 && k.spread_runs2d[gg.m]) {
       // a tile copy per wavefront while they fit 64 KB
       if (lds * kRunWaves2d > 64 * 1024) {
@@ -1834,10 +1872,25 @@ void launch_spread(const cplx<R> *f, cplx<R> *g, const Engine<R> &e, hipStream_t
   const BinGeom &gg = gb ? *gb : e.geom;
   size_t lds;
   int threads;
-  auto fn = pick_bkernel<R>(bkernels<R>(), gg, true, e.spread_variant, lds, threads);
-  // the scratch reduction needs an LDS tile; the global variant adds directly
-  if (!tiles) tiles = (lds > 0 && e.tile_scratch) ? e.tiles : nullptr;
-  if (nb > 1 && gg.d == 2 && e.spread_variant == 14 && tiles && gg.zoned &&
+  const bool shared_poly = e.win.poly_shared != 0;
+  // items of more nodes than kMx2dOneSum per wavefront
+  const bool two_sums = e.spread_max_per_sub > kMx2dOneSum * kMx2dWaves<R> || e.spread_max_items > 0;
+  auto fn = pick_bkernel<R>(bkernels<R>(), gg, true, e.spread_variant, lds, threads, shared_poly,
+                            two_sums);
+  const int blocks = mx2d_blocks(gg, e.spread_variant);
+  // the scratch reduction needs a tile per item; the global variant adds directly
+  if (!tiles) tiles = ((lds > 0 || blocks) && e.tile_scratch) ? e.tiles : nullptr;
+  if (nb > 1 && blocks == 2 && !two_sums) {
+    // as below, kMx2dRhs right-hand sides per workgroup
+    BinGeom gm = gg;
+    gm.nrhs = nb;
+    hipLaunchKernelGGL(bkernels<R>().spread_mx2d_mc[shared_poly ? 1 : 0][gg.m],
+                       dim3((unsigned)e.sp_nsub, (unsigned)((nb + kMx2dRhs - 1) / kMx2dRhs)),
+                       dim3(threads), 0, s, f, g, e.perm, e.cell, e.frac, e.sp_subs, gm, e.win,
+                       tiles);
+    return;
+  }
+  if (nb > 1 && gg.d == 2 && e.spread_variant >= 14 && tiles && gg.zoned &&
       fn == bkernels<R>().spread_runs2d[gg.m] && lds * kRhsPerGroup <= 64 * 1024 &&
       bkernels<R>().spread_runs2d_mc[gg.m]) {
     // 2-D batches: kRhsPerGroup right-hand sides per workgroup share the
@@ -1856,8 +1909,8 @@ void launch_spread(const cplx<R> *f, cplx<R> *g, const Engine<R> &e, hipStream_t
 
 // Whether the batched launches above cover this plan: the kernels that read
 // their right-hand side from blockIdx.y are the FP32 defaults (lane-per-node
-// interpolation, the run-merging spreading kernels with scratch tiles) and
-// the zone reduction.
+// interpolation, the run-merging and the 2-D matrix-core spreading kernels with
+// scratch tiles) and the zone reduction.
 template <typename R>
 bool batch_kernels(const Engine<R> &e) {
   if constexpr (!std::is_same_v<R, float>) {
@@ -1870,7 +1923,7 @@ bool batch_kernels(const Engine<R> &e) {
     if (gg.d == 3)
       return (e.spread_variant == 10 && bkernels<R>().spread_runs_2sbc[gg.m]) ||
              (e.spread_variant == 13 && bkernels<R>().spread_runs_2rs[gg.m]);
-    if (gg.d == 2) return e.spread_variant == 14 && bkernels<R>().spread_runs2d[gg.m];
+    if (gg.d == 2) return e.spread_variant >= 14 && bkernels<R>().spread_runs2d[gg.m];
     return false;
   }
 }
