@@ -25,8 +25,8 @@
 // 5.5 cycles each between FP32 products), so the kernels are built to issue
 // few of them per node.  Measured against the LDS-tile kernels (spread_impl.hpp,
 // spread_runs.hpp), m = 4, 256^3 grid:
-//   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.80 + 0.36 (reduction)
-//   B^T, FP64, 2^21 uniform nodes     3.49 + 1.87 ms -> 0.75 + 0.60
+//   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.80 + 0.26 (reduction)
+//   B^T, FP64, 2^21 uniform nodes     3.49 + 1.87 ms -> 0.75 + 0.50
 //   B,   FP64, 2^21 uniform nodes     7.03 ms -> 0.96
 //   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.53 (k_mx_interp3s)
 // FP32 sums are cut so that no product sums more than 128 nodes (B^T) or the 16
@@ -655,12 +655,20 @@ __global__ __launch_bounds__(256) void k_mx_sum3(cplx<R> *__restrict__ tiles,
 // rows.  Tile rows of 16 cells are read whole by one workgroup, so each tile
 // plane is read by the three workgroups of its dimension-1 neighbourhood
 // only; these are adjacent in the launch order of one XCD and meet in its L2.
+// Bound: the latency of bin information -> tile values, so the next bins'
+// information and the values of CH neighbours along dimension 2 are in flight
+// together.  One neighbour at a time -> as it is: 256^3 FP64, 2^21 uniform
+// nodes 595 -> 495 us (1.9 GB read, 0.27 GB written); 256^3 FP32 kooshball 319 ->
+// 219; 180 x 150 x 120 FP32 100 -> 46 (also by workgroups of 128 threads, which
+// rows of 120 cells fill).
 template <typename R, int W>
 __global__ __launch_bounds__(256) void k_mx_gather3(const cplx<R> *__restrict__ tiles,
                                                     const int4 *__restrict__ bin_info,
                                                     cplx<R> *__restrict__ g, BinGeom gg,
                                                     int chunks, int total) {
   constexpr int ROWS = 17 - W;
+  // dimension-2 neighbours whose values are in flight together
+  constexpr int CH = ROWS * sizeof(R) <= 72 ? 3 : 1;
   tiles += (long)blockIdx.y * gg.bs_t;
   g += (long)blockIdx.y * gg.bs_g;
   // consecutive work of one XCD is consecutive in (plane, bin)
@@ -672,7 +680,7 @@ __global__ __launch_bounds__(256) void k_mx_gather3(const cplx<R> *__restrict__ 
   const int b1 = w % gg.nb[1], c0 = w / gg.nb[1];
   const int n0 = gg.n[0], n1 = gg.n[1], n2 = gg.n[2];
   const int nb1 = gg.nb[1], nb2 = gg.nb[2], nb0 = gg.nb[0];
-  const int c2 = ch * 256 + threadIdx.x;
+  const int c2 = ch * (int)blockDim.x + threadIdx.x;
   if (c2 >= n2) return;
   const int lo1 = mx_lo(b1, n1, nb1), rows = mx_lo(b1 + 1, n1, nb1) - lo1;
   const int b2 = mx_bin(c2, n2, nb2);
@@ -688,38 +696,67 @@ __global__ __launch_bounds__(256) void k_mx_gather3(const cplx<R> *__restrict__ 
   R ar[ROWS], ai[ROWS];
 #pragma unroll
   for (int i = 0; i < ROWS; i++) ar[i] = ai[i] = R(0);
-  for (int j1 = 0; j1 < s1; j1++) {
-    const int bb1 = nbr(b1, j1, s1, nb1);
-    int e1 = lo1 - mx_lo(bb1, n1, nb1) + gg.m;  // tile row of the first owned row
-    e1 += e1 < 0 ? n1 : (e1 >= n1 ? -n1 : 0);
-    for (int j0 = 0; j0 < s0; j0++) {
-      const int bb0 = nbr(bB, j0, s0, nb0);
+  // tile column of this cell in the dimension-2 neighbours j2 .. j2 + CH - 1,
+  // 16 or more where the cell lies outside
+  int bb2[CH], e2[CH];
+  for (int j2 = 0; j2 < s2; j2 += CH) {
+#pragma unroll
+    for (int u = 0; u < CH; u++) {
+      e2[u] = 16;
+      bb2[u] = 0;
+      if (j2 + u < s2) {
+        bb2[u] = nbr(b2, j2 + u, s2, nb2);
+        e2[u] = c2 - mx_lo(bb2[u], n2, nb2) + gg.m;
+        e2[u] += e2[u] < 0 ? n2 : (e2[u] >= n2 ? -n2 : 0);
+      }
+    }
+    // the dimension-1 and -0 neighbours (j1, j0), a step ahead
+    int e1 = 0, e1_next = 0;
+    int4 bi[CH], bi_next[CH];
+    auto fetch = [&](int it) {
+      const int j1 = it / s0, j0 = it - j1 * s0;
+      const int bb1 = nbr(b1, j1, s1, nb1), bb0 = nbr(bB, j0, s0, nb0);
+      e1_next = lo1 - mx_lo(bb1, n1, nb1) + gg.m;  // tile row of the first owned row
+      e1_next += e1_next < 0 ? n1 : (e1_next >= n1 ? -n1 : 0);
       // planes of that bin: none beyond its cells' windows
       const int f0 = bb0 * gg.bs[0], h0 = min(n0, f0 + gg.bs[0]) - f0;
       int d0 = c0 - f0 + gg.m;
       d0 += d0 < 0 ? n0 : (d0 >= n0 ? -n0 : 0);
-      if (d0 >= h0 + W - 1) continue;
-      for (int j2 = 0; j2 < s2; j2++) {
-        const int bb2 = nbr(b2, j2, s2, nb2);
-        int e2 = c2 - mx_lo(bb2, n2, nb2) + gg.m;
-        e2 += e2 < 0 ? n2 : (e2 >= n2 ? -n2 : 0);
-        if (e2 >= 16) continue;
-        const int4 bi = bin_info[(bb1 * nb2 + bb2) * nb0 + bb0];
-        int pl = c0 - bi.y + gg.m;
+#pragma unroll
+      for (int u = 0; u < CH; u++) {
+        bi_next[u] = make_int4(0, 0, 0, 0);
+        if (d0 < h0 + W - 1 && e2[u] < 16)
+          bi_next[u] = bin_info[(bb1 * nb2 + bb2[u]) * nb0 + bb0];
+      }
+    };
+    fetch(0);
+    for (int it = 0; it < s1 * s0; it++) {
+      e1 = e1_next;
+#pragma unroll
+      for (int u = 0; u < CH; u++) bi[u] = bi_next[u];
+      if (it + 1 < s1 * s0) fetch(it + 1);
+      cplx<R> v[CH][ROWS];
+#pragma unroll
+      for (int u = 0; u < CH; u++) {
+        int pl = c0 - bi[u].y + gg.m;
         pl += pl < 0 ? n0 : (pl >= n0 ? -n0 : 0);
-        if (pl >= bi.z) continue;
-        const cplx<R> *tp = tiles + ((long)bi.x + pl) * 256 + e2;
+        const bool in = pl < bi[u].z;
+        const cplx<R> *tp = tiles + ((long)bi[u].x + pl) * 256 + e2[u];
 #pragma unroll
         for (int i = 0; i < ROWS; i++) {
           int e = e1 + i;
           e -= e >= n1 ? n1 : 0;
-          if (e < 16 && i < rows) {
-            const cplx<R> v = tp[e * 16];
-            ar[i] += v.x;
-            ai[i] += v.y;
-          }
+          v[u][i] = cplx<R>{0, 0};
+          if (in && e < 16 && i < rows) v[u][i] = tp[e * 16];
         }
       }
+#pragma unroll
+      for (int u = 0; u < CH; u++)
+#pragma unroll
+        for (int i = 0; i < ROWS; i++) {
+          ar[i] += v[u][i].x;
+          ai[i] += v[u][i].y;
+        }
     }
   }
   cplx<R> *gp = g + ((long)c0 * n1 + lo1) * n2 + c2;
@@ -763,10 +800,11 @@ void mx_gather3(const cplx<R> *tiles, cplx<R> *g, const Engine<R> &e, const BinG
                        dim3(256), 0, s, const_cast<cplx<R> *>(tiles), e.mx_info, e.mx_bin_info,
                        e.mx_multi, e.sp_first, e.sp_count, gg);
   const int chunks = (gg.n[2] + 255) / 256;
+  const int threads = (gg.n[2] + 64 * chunks - 1) / (64 * chunks) * 64;  // of 256 at most
   const int total = gg.n[0] * gg.nb[1] * chunks;
   const unsigned blocks = 8u * (unsigned)((total + 7) / 8);
-  hipLaunchKernelGGL((k_mx_gather3<R, 2 * M_ + 2>), dim3(blocks, (unsigned)nb), dim3(256), 0, s,
-                     tiles, e.mx_bin_info, g, gg, chunks, total);
+  hipLaunchKernelGGL((k_mx_gather3<R, 2 * M_ + 2>), dim3(blocks, (unsigned)nb),
+                     dim3((unsigned)threads), 0, s, tiles, e.mx_bin_info, g, gg, chunks, total);
 }
 
 // the launches of window cut-off m (1 .. kMxMaxM)
