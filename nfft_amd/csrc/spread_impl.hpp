@@ -1534,25 +1534,34 @@ __global__ __launch_bounds__(256) void k_gather_zones(const cplx<R> *__restrict_
   }
 }
 
+// right-hand sides of a batch per workgroup of the reduction below
+constexpr int kZoneRhs = 4;
+
 // The same reduction for d = 1, 2: a thread owns one core cell and knows its
 // place in each of the 3^d zones, so that the loop over the items has no lists
 // or tables in LDS, and up to U items of all neighbours are in flight at once.
 // `parts` workgroups share a bin.  Bound: the chain order -> first item -> tile
 // values -> grid cell, and in dense regions a load more per U items of a bin.
 // 512^2 grid, 128512 radial nodes in 987 items, some 60 in the heaviest
-// neighbourhood: 17 us with k_gather_zones, 9 here.
-template <typename R, int D>
+// neighbourhood: 17 us with k_gather_zones, 7 here; 32 right-hand sides of
+// 206336 such nodes 138 -> 74, 1-D 2^22 cells 30 -> 23.
+//
+// PAIR: the bin edges are 2m + 1 cells or more, so that a cell lies in the own
+// zone and at most one neighbour's per dimension (of bins of 16 cells, m = 4:
+// four places to look instead of nine).  A workgroup takes RH right-hand sides
+// of a batch, its addresses computed once.
+template <typename R, int D, bool PAIR>
 __global__ __launch_bounds__(256) void k_gather_zones_cell(const cplx<R> *__restrict__ tiles,
                                                            const int *__restrict__ sp_first,
                                                            const int *__restrict__ sp_count,
                                                            cplx<R> *__restrict__ g, BinGeom gg,
                                                            const int *__restrict__ order,
-                                                           int parts) {
+                                                           int parts, int nrhs) {
   static_assert(D == 1 || D == 2, "3-D: k_gather_zones");
-  constexpr int NZ = D == 1 ? 3 : 9, U = 2;
-  // right-hand side blockIdx.y of a batched launch
-  tiles += (long)blockIdx.y * gg.bs_t;
-  g += (long)blockIdx.y * gg.bs_g;
+  constexpr int ND = PAIR ? 2 : 3, NZ = D == 1 ? ND : ND * ND, U = PAIR ? 4 : 2;
+  const int r0 = blockIdx.y * kZoneRhs, rn = min(nrhs - r0, kZoneRhs);
+  tiles += (long)r0 * gg.bs_t;
+  g += (long)r0 * gg.bs_g;
   const int bin = order[blockIdx.x / parts];  // heavy neighbourhoods first
   // (1-D: as a second dimension of one bin and cell)
   const int nb1 = D == 2 ? gg.nb[1] : 1, bs1 = D == 2 ? gg.bs[1] : 1;
@@ -1561,41 +1570,53 @@ __global__ __launch_bounds__(256) void k_gather_zones_cell(const cplx<R> *__rest
   const int core = gg.bs[0] * bs1;
   const int q = (int)(blockIdx.x % parts) * 256 + threadIdx.x;
   const int k0 = q / bs1, k1 = q - k0 * bs1;
+  // neighbour digit (0 left, 1 self, 2 right) of choice i along a dimension,
+  // and whether its zone (the left one's m + 1 last cells, the right one's m
+  // first) holds cell k
+  auto digit = [&](int i, int k, int bs) { return !PAIR ? i : (i == 0 ? 1 : (k <= gg.m ? 0 : 2)); };
+  auto inside = [&](int dg, int k, int bs) {
+    return dg == 1 || (dg == 0 ? k <= gg.m : k >= bs - gg.m);
+  };
   const cplx<R> *tp[NZ];
   int cnt[NZ], most = 0;
 #pragma unroll
   for (int z = 0; z < NZ; z++) {
-    int v0 = b0 + (D == 2 ? z / 3 : z) - 1, v1 = D == 2 ? b1 + z % 3 - 1 : 0;
+    const int g0 = digit(D == 2 ? z / ND : z, k0, gg.bs[0]), g1 = D == 2 ? digit(z % ND, k1, bs1) : 1;
+    int v0 = b0 + g0 - 1, v1 = b1 + g1 - 1;
     v0 += v0 < 0 ? gg.nb[0] : (v0 >= gg.nb[0] ? -gg.nb[0] : 0);
     v1 += v1 < 0 ? nb1 : (v1 >= nb1 ? -nb1 : 0);
     const int nbl = v0 * nb1 + v1, n = sp_count[nbl];
-    const int *zd = gg.zdesc + 8 * z;  // its zone's place in the tile and in this core
-    const int u0 = k0 - zd[1], u1 = D == 2 ? k1 - zd[2] : 0;
-    const bool in = q < core && u0 >= 0 && u0 < zd[4] && (D == 1 || (u1 >= 0 && u1 < zd[5]));
+    const int *zd = gg.zdesc + 8 * (D == 2 ? 3 * g0 + g1 : g0);  // the zone's place in the tile
+    const int u0 = g0 == 2 ? k0 - gg.bs[0] + gg.m : k0, u1 = g1 == 2 ? k1 - bs1 + gg.m : k1;
+    const int w1 = g1 == 1 ? bs1 : (g1 == 0 ? gg.m + 1 : gg.m);
+    const bool in = q < core && inside(g0, k0, gg.bs[0]) && (D == 1 || inside(g1, k1, bs1));
     cnt[z] = in ? n : 0;
-    most = max(most, n);
-    tp[z] = tiles + (long)sp_first[nbl] * tot + zd[0] + (D == 2 ? u0 * zd[5] + u1 : u0);
+    most = max(most, cnt[z]);
+    tp[z] = tiles + (long)sp_first[nbl] * tot + zd[0] + (D == 2 ? u0 * w1 + u1 : u0);
   }
-  R ar = 0, ai = 0;
-  for (int c = 0; c < most; c += U) {
-    cplx<R> v[U][NZ];
+  cplx<R> *gp = g + (long)(b0 * gg.bs[0] + k0) * (D == 2 ? gg.n[1] : 1) + b1 * bs1 + k1;
+  for (int r = 0; r < rn; r++) {
+    const long rt = (long)r * gg.bs_t;
+    R ar = 0, ai = 0;
+    for (int c = 0; c < most; c += U) {
+      cplx<R> v[U][NZ];
 #pragma unroll
-    for (int u = 0; u < U; u++)
+      for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int z = 0; z < NZ; z++) {
-        v[u][z] = cplx<R>{0, 0};
-        if (c + u < cnt[z]) v[u][z] = tp[z][(long)(c + u) * tot];
-      }
+        for (int z = 0; z < NZ; z++) {
+          v[u][z] = cplx<R>{0, 0};
+          if (c + u < cnt[z]) v[u][z] = tp[z][rt + (long)(c + u) * tot];
+        }
 #pragma unroll
-    for (int u = 0; u < U; u++)
+      for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int z = 0; z < NZ; z++) {
-        ar += v[u][z].x;
-        ai += v[u][z].y;
-      }
+        for (int z = 0; z < NZ; z++) {
+          ar += v[u][z].x;
+          ai += v[u][z].y;
+        }
+    }
+    if (q < core) gp[(long)r * gg.bs_g] = cplx<R>{ar, ai};
   }
-  if (q < core)
-    g[(long)(b0 * gg.bs[0] + k0) * (D == 2 ? gg.n[1] : 1) + b1 * bs1 + k1] = cplx<R>{ar, ai};
 }
 
 // zone reduction of nb right-hand sides
@@ -1609,9 +1630,12 @@ void launch_gather_zones(const cplx<R> *tiles, const Engine<R> &e, cplx<R> *g, c
   }
   if (gg.d <= 2) {
     const int parts = (int)((core + 255) / 256);
-    auto fn = gg.d == 1 ? k_gather_zones_cell<R, 1> : k_gather_zones_cell<R, 2>;
-    hipLaunchKernelGGL(fn, dim3((unsigned)(nbins * parts), (unsigned)nb), dim3(256), 0, s, tiles,
-                       e.sp_first, e.sp_count, g, gg, e.bin_order, parts);
+    bool pair = true;
+    for (int t = 0; t < gg.d; t++) pair = pair && gg.bs[t] >= 2 * gg.m + 1;
+    auto fn = gg.d == 1 ? (pair ? k_gather_zones_cell<R, 1, true> : k_gather_zones_cell<R, 1, false>)
+                        : (pair ? k_gather_zones_cell<R, 2, true> : k_gather_zones_cell<R, 2, false>);
+    hipLaunchKernelGGL(fn, dim3((unsigned)(nbins * parts), (unsigned)((nb + kZoneRhs - 1) / kZoneRhs)),
+                       dim3(256), 0, s, tiles, e.sp_first, e.sp_count, g, gg, e.bin_order, parts, nb);
     return;
   }
   // one workgroup per bin (two measured slower on the kooshball: 0.25 -> 0.33 ms)
