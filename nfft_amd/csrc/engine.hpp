@@ -313,7 +313,7 @@ template <typename R> struct Engine {
   cplx<R> *grid_after_trafo() const { return trafo_grid ? g2 : g; }
 
   void create(int d_, const long *N_, const long *n_, long M_, int m_);
-  void set_bins(const int *bs);
+  void set_bins(const int *bs, bool tables = true);
   void set_mx_bins();
   void set_mx2d_bins();
   void destroy();

@@ -159,8 +159,11 @@ __global__ void k_bins_from_keys(const int *__restrict__ kstart, long nbins, int
 // occupied cells: positions where the sorted key changes
 __global__ __launch_bounds__(256) void k_count_cells(const unsigned *__restrict__ key, long M,
                                                      int *__restrict__ count) {
-  const long j = (long)blockIdx.x * 256 + threadIdx.x;
-  const int n = __popcll(__ballot(j < M && (j == 0 || key[j] != key[j - 1])));
+  int n = 0;  // (whole wavefronts take every turn)
+  for (long j0 = (long)blockIdx.x * 256; j0 < M; j0 += (long)gridDim.x * 256) {
+    const long j = j0 + threadIdx.x;
+    n += __popcll(__ballot(j < M && (j == 0 || key[j] != key[j - 1])));
+  }
   __shared__ int sum[4];
   if ((threadIdx.x & 63) == 0) sum[threadIdx.x >> 6] = n;
   __syncthreads();
@@ -635,7 +638,7 @@ void bin_nodes(Engine<R> &e) {
   if (gg.mx && sizeof(R) == 4 && M > 0) {
     int cells = 0;
     launch_fill_zero_int(sums + 1, 1, s);
-    hipLaunchKernelGGL(k_count_cells, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s, key_sorted,
+    hipLaunchKernelGGL(k_count_cells, dim3((unsigned)std::min(2048L, ceil_div(M, 256))), dim3(256), 0, s, key_sorted,
                        M, sums + 1);
     NFFT_HIP_CHECK(R, hipMemcpyAsync(&cells, sums + 1, sizeof(int), hipMemcpyDeviceToHost, s));
     NFFT_HIP_CHECK(R, hipStreamSynchronize(s));

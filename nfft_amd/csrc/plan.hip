@@ -272,9 +272,10 @@ static void spread_lane_table(int W, int gc, int E0, int E1, int E2, int &pp_out
 // Bin edges bs[t] (and with them the LDS tile edge bs + 2m + 1): the
 // geometry shared by the node binning and the B / B^T kernels, whether B^T
 // reduces its tiles through scratch, and the zone tables of that reduction.
-// Node data must be rebuilt after a change (build_nodes).
+// Node data must be rebuilt after a change (build_nodes).  tables = false: the
+// geometry alone, for bins that may still be replaced.
 template <typename R>
-void Engine<R>::set_bins(const int *bs) {
+void Engine<R>::set_bins(const int *bs, bool tables) {
   geom.d = d;
   geom.m = m;
   geom.M = M;
@@ -342,7 +343,7 @@ void Engine<R>::set_bins(const int *bs) {
     geom.zmap = geom.zdesc = nullptr;
     if (zone_tab) NFFT_HIP_CHECK(R, hipFree(zone_tab));
     zone_tab = nullptr;
-    if (zoned) {
+    if (zoned && tables) {
       // per dimension the tile splits into the part in the left neighbour's
       // core (m cells), the own core (bs), the part in the right
       // neighbour's core (m + 1); zones are written in base-3 order of
@@ -590,7 +591,7 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
       if (*q == ',') q++;
     }
   }
-  set_bins(bs);
+  set_bins(bs, false);
   // nodes per work item; larger 3-D spreading items write fewer tiles for
   // the reduction (measured on the 3-D kooshball: 2048 -> 4096 halves the
   // tile reduction at equal spreading time, larger items end the launch late)
@@ -635,6 +636,7 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
 
   set_mx_bins();
   if (!std::getenv("NFFT_HIP_BINS")) set_mx2d_bins();
+  if (geom.zoned && !zone_tab) set_bins(bs);
 
   // FFT: twiddles per dimension, then the pruned passes of both directions.
   // An axis whose lines fit one workgroup's LDS (cap elements) and whose
