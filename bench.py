@@ -572,9 +572,9 @@ def main():
     b_trafo_ms = stages_ms["trafo_B"]
     b_adj_ms = stages_ms["adjoint_B"]
     if b_adj_ms >= b_trafo_ms:
-        dom_name, dom_ms, dom_sym = "B^T spreading (k_spread_runs, adjoint)", b_adj_ms, "k_spread_runs"
+        dom_name, dom_ms, dom_sym = "B^T spreading (k_mx_spread3, adjoint)", b_adj_ms, "k_mx_spread3"
     else:
-        dom_name, dom_ms, dom_sym = "B interpolation (k_interp_tile, trafo)", b_trafo_ms, "k_interp_tile"
+        dom_name, dom_ms, dom_sym = "B interpolation (k_mx_interp3s, trafo)", b_trafo_ms, "k_mx_interp3s"
     # HBM bytes per launch of that kernel measured by rocprofv3 FETCH_SIZE /
     # WRITE_SIZE (copy-calibrated) and committed with the profile summaries
     # (the profile names the exact kernel each stage ran in its run)
@@ -583,7 +583,7 @@ def main():
     if os.path.exists(tpath):
         with open(tpath) as fh_:
             tj = json.load(fh_)
-        stage = "adjoint_B" if dom_sym == "k_spread_runs" else "trafo_B"
+        stage = "adjoint_B" if dom_sym == "k_mx_spread3" else "trafo_B"
         kname = tj.get("stage_kernels", {}).get(stage)
         if kname in tj.get("kernels", {}):
             traffic = tj["kernels"][kname]["traffic_bytes"]
