@@ -1652,17 +1652,19 @@ void launch_gather_tiles(const Engine<R> &e, cplx<R> *g, hipStream_t s, int nb, 
     launch_mx_gather<R>(e, g, s, nb, gb, tiles);
     return;
   }
-  long nbins = 1;
-  for (int t = 0; t < e.geom.d; t++) nbins *= e.geom.nb[t];
+  // the tiles that launch_spread wrote: the caller's, also for a chunk of one
+  // right-hand side of a batch
+  const BinGeom &gg = gb ? *gb : e.geom;
+  if (!tiles) tiles = e.tiles;
   // (only zoned plans run batches in one launch)
-  if (nb > 1 || e.geom.zoned) {
-    launch_gather_zones<R>(nb > 1 ? tiles : e.tiles, e, g, nb > 1 ? *gb : e.geom, s, nb);
+  if (gg.zoned) {
+    launch_gather_zones<R>(tiles, e, g, gg, s, nb);
     return;
   }
-  auto fn = e.geom.d == 1 ? k_gather_tiles<R, 1> : e.geom.d == 2 ? k_gather_tiles<R, 2>
-                                                                 : k_gather_tiles<R, 3>;
-  hipLaunchKernelGGL(fn, dim3((unsigned)nbins), dim3(256), 0, s, e.tiles, e.sp_first, e.sp_count,
-                     g, e.geom);
+  long nbins = 1;
+  for (int t = 0; t < gg.d; t++) nbins *= gg.nb[t];
+  auto fn = gg.d == 1 ? k_gather_tiles<R, 1> : gg.d == 2 ? k_gather_tiles<R, 2> : k_gather_tiles<R, 3>;
+  hipLaunchKernelGGL(fn, dim3((unsigned)nbins), dim3(256), 0, s, tiles, e.sp_first, e.sp_count, g, gg);
 }
 
 // ==================================================================== dispatch
