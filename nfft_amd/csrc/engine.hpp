@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "mx_index.hpp"
 
 namespace nfft_hip {
 
@@ -77,11 +78,6 @@ struct BinGeom {
 // the library's static scratch for allocation-free batched adjoints (plan.hip)
 constexpr long kNoAllocScratchBytes = 64L << 20;
 
-// Ragged bins: first cell of bin b of nb over n cells, and the bin of cell c
-// (n <= kMxMaxN, so that the products fit an int)
-constexpr int kMxMaxN = 32767;
-__host__ __device__ inline int mx_lo(int b, int n, int nb) { return b * n / nb; }
-__host__ __device__ inline int mx_bin(int c, int n, int nb) { return ((c + 1) * nb - 1) / n; }
 // 2-D matrix-core B^T (spread_mx2d.hpp): widest tile and window, wavefronts per
 // item, right-hand sides per workgroup of a batch, nodes summed in FP32 before
 // the sums are summed
@@ -90,8 +86,6 @@ constexpr int kMx2dMaxM = 8;
 template <typename R> constexpr int kMx2dWaves = sizeof(R) == 4 ? 4 : 2;
 constexpr int kMx2dRhs = 2;
 constexpr int kMx2dOneSum = 64;
-// widest window of the 3-D matrix-core kernels: m = kMxMaxM
-constexpr int kMxMaxM = 6;
 
 // Kaiser-Bessel window of one dimension, scaled by 1/phi(0) so that the B
 // weights stay O(1) (the scale is folded into the deconvolution factors).

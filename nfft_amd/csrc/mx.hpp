@@ -210,7 +210,6 @@ __global__ __launch_bounds__(128, sizeof(R) == 4 ? (W <= 10 ? 4 : 3) : 2) void k
 // and loads each plane once as the nodes move on (the next one ahead of its
 // use).  FP32: both parts in one wavefront; FP64: the real parts in one, the
 // imaginary parts in the other.
-constexpr int kMxSpan = 4;
 template <typename R> constexpr int kMxParts = sizeof(R) == 4 ? 1 : 2;
 
 template <typename R, int W, bool SHARED>
@@ -219,7 +218,7 @@ __global__ __launch_bounds__(64 * kMxParts<R>, sizeof(R) == 4 && W <= 10 ? 3 : 2
     const int *__restrict__ cell, const R *__restrict__ frac, const int4 *__restrict__ subs,
     BinGeom gg, WinParams<R> wp) {
   constexpr int NW = kMxParts<R>, NP = 2 / NW, NC = 16 * NW;
-  constexpr int Z = kMxSpan - 1, RW = W + Z;
+  constexpr int Z = kMxSpan - 1, RW = mx_ring(W);
   static_assert(W + 2 * Z <= kMxPitch, "zeros before and after the dimension-0 taps");
   // window rows: dimension 1, 0 (taps from position Z on), 2.  (A lane whose
   // node is not of the cells at hand reads outside its dimension-0 row, at
@@ -257,9 +256,7 @@ __global__ __launch_bounds__(64 * kMxParts<R>, sizeof(R) == 4 && W <= 10 ? 3 : 2
   }
   const long plane = (long)gg.n[1] * gg.n[2];
   auto load_plane = [&](int p, R (&d)[NP][4]) {
-    int c0 = p - gg.m;
-    c0 += c0 < 0 ? gg.n[0] : 0;
-    c0 -= c0 >= gg.n[0] ? gg.n[0] : 0;
+    const int c0 = mx_plane(p, gg.m, gg.n[0]);
     const cplx<R> *gp = g + (long)c0 * plane;
 #pragma unroll
     for (int s = 0; s < 4; s++) {
@@ -443,9 +440,7 @@ __global__ __launch_bounds__(64, 2) void k_mx_interp3s(
   }
   const long plane = (long)gg.n[1] * gg.n[2];
   auto load_plane = [&](int p, float2 (&d)[4]) {
-    int c0 = p - gg.m;
-    c0 += c0 < 0 ? gg.n[0] : 0;
-    c0 -= c0 >= gg.n[0] ? gg.n[0] : 0;
+    const int c0 = mx_plane(p, gg.m, gg.n[0]);
     const float2 *gp = g + (long)c0 * plane;
 #pragma unroll
     for (int s = 0; s < 4; s++) d[s] = gp[goff[s]];
