@@ -279,6 +279,7 @@ template <typename R> struct Engine {
   size_t aux_cap = 0;
   long scratch_cap = 0;
   bool nodes_ready = false;
+  long node_builds = 0;  // changes with the node data (a captured launch holds their sizes)
 
   BinGeom geom{};
   WinParams<R> win{};

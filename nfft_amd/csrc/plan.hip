@@ -876,6 +876,7 @@ void Engine<R>::build_nodes() {
     }
   }
   nodes_ready = true;
+  node_builds++;
 }
 
 // events bracketing the stages of one call: the immediate set, a fresh set

@@ -197,11 +197,13 @@ template <typename R> struct DevCgnr {
   // The kernels of one step (everything but the copies back to the host)
   // as a hipGraph, captured on the first step and replayed with one launch
   // afterwards (NFFT_HIP_CGNR_GRAPH=0 at solver creation: eager launches).
-  // Re-captured when the plan's stream changes; not used while stage timing
-  // is on (its events are created on demand).
+  // Re-captured when the plan's stream or its node data change (the launches
+  // hold item counts, list addresses and the choice of kernels); not used
+  // while stage timing is on (its events are created on demand).
   bool use_graph = true;
   hipGraphExec_t step_exec = nullptr;
   hipStream_t step_stream = nullptr;
+  long step_builds = 0;
 
   void alloc(Engine<R> *eng, long M_, long N_, bool weighted, bool damped) {
     e = eng;
@@ -427,7 +429,7 @@ struct SolverApi {
     Engine<R> *e = dv->e;
     hipStream_t s = e->stream;
     if (dv->use_graph && !e->timing && !e->deferred) {
-      if (!dv->step_exec || dv->step_stream != s) {
+      if (!dv->step_exec || dv->step_stream != s || dv->step_builds != e->node_builds) {
         if (dv->step_exec) NFFT_HIP_CHECK(R, hipGraphExecDestroy(dv->step_exec));
         dv->step_exec = nullptr;
         hipGraph_t graph;
@@ -437,6 +439,7 @@ struct SolverApi {
         NFFT_HIP_CHECK(R, hipGraphInstantiate(&dv->step_exec, graph, nullptr, nullptr, 0));
         NFFT_HIP_CHECK(R, hipGraphDestroy(graph));
         dv->step_stream = s;
+        dv->step_builds = e->node_builds;
       }
       NFFT_HIP_CHECK(R, hipGraphLaunch(dv->step_exec, s));
     } else {
