@@ -243,7 +243,6 @@ template <typename R> struct Engine {
   // the same per spreading bin (z = 0: no nodes): its item's, or for a bin of
   // several items those of the tile their planes are summed into; the bins of
   // several items
-  bool mx_dense = false;  // several nodes per occupied cell: see bin_nodes
   int4 *mx_bin_info = nullptr;
   int *mx_multi = nullptr;
   long mx_bins_cap = 0, mx_multi_n = 0;

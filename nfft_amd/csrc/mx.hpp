@@ -28,7 +28,7 @@
 //   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.80 + 0.26 (reduction)
 //   B^T, FP64, 2^21 uniform nodes     3.49 + 1.87 ms -> 0.75 + 0.50
 //   B,   FP64, 2^21 uniform nodes     7.03 ms -> 0.96
-//   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.53 (k_mx_interp3s)
+//   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.96
 // FP32 sums are cut so that no product sums more than 128 nodes (B^T) or the 16
 // positions of one plane (B): single sums over an item or a window lost up to a
 // bit (kooshball adjoint 3.0e-7 against FP64, 2.1e-7 as it is and before).
@@ -365,232 +365,6 @@ __global__ __launch_bounds__(64 * kMxParts<R>, sizeof(R) == 4 && W <= 10 ? 3 : 2
   }
 }
 
-// B in FP32 on the bf16 products, whose rate is eight times that of the FP32
-// ones and which leave the vector ALUs free.  Grid values and weights are
-// split into three bf16 pieces each (8 + 8 + 8 bits: the pieces' sum is the
-// FP32 value), and the six products of pieces above 2^-24 of the largest are
-// summed in FP32: g w = gh wh + (gh wm + gm wh) + (gh wl + gm wm + gl wh).
-// One 16 x 16 x 32 product takes two of them over the 16 columns e2, so a plane
-// and part takes three; the planes are summed with the FP32 weights psi0 by the
-// vector ALUs,
-//   C[e1][k] += psi0_k[i] (sum_e2 g_i[e1][e2] psi2_k[e2]).
-using mx_bf2 = __bf16 __attribute__((ext_vector_type(2)));
-using mx_bf8 = __bf16 __attribute__((ext_vector_type(8)));
-using mx_f2 = float __attribute__((ext_vector_type(2)));
-using mx_u6 = unsigned __attribute__((ext_vector_type(6)));
-using mx_u4 = unsigned __attribute__((ext_vector_type(4)));
-
-// x = h + m + l in bf16 pieces (each rounded to nearest), two values at once
-__device__ __forceinline__ void mx_split(mx_f2 x, unsigned &h, unsigned &m, unsigned &l) {
-  const mx_bf2 a = __builtin_convertvector(x, mx_bf2);
-  mx_f2 r = x - __builtin_convertvector(a, mx_f2);
-  const mx_bf2 b = __builtin_convertvector(r, mx_bf2);
-  r = r - __builtin_convertvector(b, mx_f2);
-  const mx_bf2 c = __builtin_convertvector(r, mx_bf2);
-  h = __builtin_bit_cast(unsigned, a);
-  m = __builtin_bit_cast(unsigned, b);
-  l = __builtin_bit_cast(unsigned, c);
-}
-__device__ __forceinline__ mx4<float> mx_mul16(mx_u4 a, mx_u4 b, mx4<float> c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mx_bf8, a),
-                                                 __builtin_bit_cast(mx_bf8, b), c, 0, 0, 0);
-}
-
-// The form for dense node sets (three nodes or more per occupied cell): 32
-// nodes of up to two dimension-0 cells at a time share the ring's planes,
-// without a branch per plane.  On the 3-D kooshball 1.53 ms against 1.96 for
-// k_mx_interp3 and 1.62 for the LDS-tile kernel; on 0.09 nodes per cell
-// k_mx_interp3 is the faster one, 0.073 against 0.087 ms.  Its error against
-// 64 bits is no larger than that of FP32 products (m = 4, 64 x 64 x 64 grid:
-// 1.5e-7 against 1.7e-7), since the pieces hold all 24 bits.  The bound is the
-// issue of its 390 instructions per 16 nodes at two wavefronts per SIMD (the
-// ring takes 132 registers).
-constexpr int kMxSpanDense = 2;
-
-template <int W, bool SHARED>
-__global__ __launch_bounds__(64, 2) void k_mx_interp3s(
-    const float2 *__restrict__ g, float2 *__restrict__ fout, const int *__restrict__ perm,
-    const int *__restrict__ cell, const float *__restrict__ frac, const int4 *__restrict__ subs,
-    BinGeom gg, WinParams<float> wp) {
-  constexpr int NC = 32, Z = kMxSpanDense - 1, RW = W + Z;
-  static_assert(W + 2 * Z <= kMxPitch, "zeros before and after the dimension-0 taps");
-  __shared__ __align__(16) float win[3 * NC * kMxPitch];  // as in k_mx_interp3
-  __shared__ __align__(16) float spoly[SHARED ? 1 : 3 * (W / 2) * kMxCoef<float>];
-  g += (long)blockIdx.y * gg.bs_g;
-  fout += (long)blockIdx.y * gg.bs_f;
-  const int4 sp = subs[blockIdx.x];
-  const int lane = threadIdx.x, j = lane & 15, q = lane >> 4;
-  const int col = sp.x / gg.nb[0];
-  const int b1 = col / gg.nb[2], b2 = col - b1 * gg.nb[2];
-  const int lo1 = mx_lo(b1, gg.n[1], gg.nb[1]), lo2 = mx_lo(b2, gg.n[2], gg.nb[2]);
-  if constexpr (!SHARED) {
-    mx_load_poly<float, 3, W>(spoly, wp.poly, threadIdx.x, 64);
-    __syncthreads();
-  }
-  unsigned goff[4];
-  {
-    int c1 = lo1 - gg.m + j;
-    c1 += c1 < 0 ? gg.n[1] : (c1 >= gg.n[1] ? -gg.n[1] : 0);
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      int c2 = lo2 - gg.m + 4 * q + s;
-      c2 += c2 < 0 ? gg.n[2] : (c2 >= gg.n[2] ? -gg.n[2] : 0);
-      goff[s] = (unsigned)c1 * gg.n[2] + c2;
-    }
-  }
-  const long plane = (long)gg.n[1] * gg.n[2];
-  auto load_plane = [&](int p, float2 (&d)[4]) {
-    const int c0 = mx_plane(p, gg.m, gg.n[0]);
-    const float2 *gp = g + (long)c0 * plane;
-#pragma unroll
-    for (int s = 0; s < 4; s++) d[s] = gp[goff[s]];
-  };
-  // a plane's pieces, per part: low, high, middle pieces of e2 = 4 q .. 4 q + 3
-  mx_u6 ring[RW][2];
-  auto put = [](mx_u6 &r, float a, float b, float c, float d) {
-    unsigned h0, m0, l0, h1, m1, l1;
-    mx_split(mx_f2{a, b}, h0, m0, l0);
-    mx_split(mx_f2{c, d}, h1, m1, l1);
-    r = mx_u6{l0, l1, h0, h1, m0, m1};
-  };
-  auto put_plane = [&](mx_u6 (&r)[2], const float2 (&d)[4]) {
-    put(r[0], d[0].x, d[1].x, d[2].x, d[3].x);
-    put(r[1], d[0].y, d[1].y, d[2].y, d[3].y);
-  };
-  int ra = cell[sp.y];  // the ring holds planes ra .. ra + RW - 1, plane p in slot p mod RW
-  int rot = ra % RW;
-  float2 next[4];
-#pragma unroll
-  for (int s = 0; s < RW; s++) {
-    float2 d[4];
-    load_plane(ra + (s < rot ? s - rot + RW : s - rot), d);
-    put_plane(ring[s], d);
-  }
-  load_plane(ra + RW, next);
-  // lane = node + 32 t evaluates dimension t = 0, 1 and, lanes below 32,
-  // dimension 2 (rows of win: dimension 1, 0, 2)
-  const int me = lane & 31, t = lane >> 5;
-  const int *cellp = cell + t * gg.M + sp.y, *cell2 = cell + 2 * gg.M + sp.y;
-  const float *fracp = frac + t * gg.M + sp.y, *frac2 = frac + 2 * gg.M + sp.y;
-  const int *permp = perm + sp.y;
-  const int last = sp.z - 1;
-  int c = cellp[min(me, last)], d2 = cell2[min(me, last)];
-  float fr = fracp[min(me, last)], fr2 = frac2[min(me, last)];
-  for (int base = 0; base < sp.z; base += NC) {
-    const int c0 = c;  // lanes 0..31: the chunk's dimension-0 cells
-    {
-      const float *poly = wp.poly;
-      asm volatile("" : "+s"(poly));  // as in k_mx_spread3
-      mx_window_row<float, W>(win + ((1 - t) * NC + me) * kMxPitch, t == 0 ? Z : c - lo1, fr - 0.5f,
-                              [&](int w) {
-                                if constexpr (SHARED) return poly + w * (kPolyDeg + 1);
-                                else return spoly + (t * (W / 2) + w) * kMxCoef<float>;
-                              });
-      if (t == 0)
-        mx_window_row<float, W>(win + (2 * NC + me) * kMxPitch, d2 - lo2, fr2 - 0.5f, [&](int w) {
-          if constexpr (SHARED) return poly + w * (kPolyDeg + 1);
-          else return spoly + (W + w) * kMxCoef<float>;
-        });
-    }
-    const int pj = permp[min(base + me, last)];
-    const int nn = min(base + NC + me, last);
-    c = cellp[nn];
-    fr = fracp[nn];
-    d2 = cell2[nn];
-    fr2 = frac2[nn];
-    __syncthreads();
-    const int cnt = min(NC, sp.z - base);
-    // weights of the nodes j and j + 16 for the piece pairs (h, m), (l, h), (h, m)
-    mx_u4 w1[2], w2[2], w3[2];
-    int cj[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const float *r2 = win + (2 * NC + 16 * h + j) * kMxPitch + 4 * q;
-      unsigned h0, m0, l0, h1, m1, l1;
-      mx_split(mx_f2{r2[0], r2[1]}, h0, m0, l0);
-      mx_split(mx_f2{r2[2], r2[3]}, h1, m1, l1);
-      w1[h] = mx_u4{h0, h1, h0, h1};
-      w2[h] = mx_u4{h0, h1, m0, m1};
-      w3[h] = mx_u4{l0, l1, m0, m1};
-      cj[h] = __shfl(c0, 16 * h + j, 64);
-    }
-    for (int k = 0; k < cnt;) {
-      // nodes k .. end - 1: cells ak .. az
-      const int ak = __builtin_amdgcn_readlane(c0, k);
-      const int end = __popcll(__ballot(lane < cnt && c0 <= ak + Z));
-      const int az = __builtin_amdgcn_readlane(c0, end - 1);
-      for (; ra < az - Z; ra++) {
-        mx_u6 nx[2];
-        put_plane(nx, next);
-#pragma unroll
-        for (int s = 0; s < RW; s++)
-          if (rot == s) {
-            ring[s][0] = nx[0];
-            ring[s][1] = nx[1];
-          }
-        rot = rot + 1 < RW ? rot + 1 : 0;
-        load_plane(ra + 1 + RW, next);
-      }
-      // planes that a node does not reach meet zeros of its row (ra <= ak and
-      // ra + Z >= az)
-      mx4<float> acc[2][2] = {};
-      const float *w0[2];
-#pragma unroll
-      for (int h = 0; h < 2; h++)
-        w0[h] = win + (NC + 16 * h + j) * kMxPitch + Z - cj[h] + ra;
-#pragma unroll
-      for (int s = 0; s < RW; s++) {
-        const int i = s < rot ? s - rot + RW : s - rot;
-        mx_u4 a[2], b[2];
-#pragma unroll
-        for (int x = 0; x < 2; x++) {
-          b[x] = __builtin_shufflevector(ring[s][x], ring[s][x], 0, 1, 2, 3);
-          a[x] = __builtin_shufflevector(ring[s][x], ring[s][x], 2, 3, 4, 5);
-        }
-        mx4<float> z[2][2] = {};
-        // small products first
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-          for (int x = 0; x < 2; x++) z[h][x] = mx_mul16(a[x], w3[h], z[h][x]);
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-          for (int x = 0; x < 2; x++) z[h][x] = mx_mul16(b[x], w2[h], z[h][x]);
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-          for (int x = 0; x < 2; x++) z[h][x] = mx_mul16(a[x], w1[h], z[h][x]);
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const float w = w0[h][i];
-#pragma unroll
-          for (int x = 0; x < 2; x++)
-#pragma unroll
-            for (int u = 0; u < 4; u++) acc[h][x][u] = fmaf(w, z[h][x][u], acc[h][x][u]);
-        }
-      }
-      float out[2][2] = {};
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const float p1 = win[(16 * h + j) * kMxPitch + 4 * q + u];
-#pragma unroll
-          for (int x = 0; x < 2; x++) out[h][x] = fmaf(acc[h][x][u], p1, out[h][x]);
-        }
-#pragma unroll
-        for (int x = 0; x < 2; x++) out[h][x] = mx_col_sum(out[h][x]);
-      }
-      // lanes 0..31: node = lane
-      if (lane >= k && lane < end)
-        fout[pj] = float2{lane < 16 ? out[0][0] : out[1][0], lane < 16 ? out[0][1] : out[1][1]};
-      k = end;
-    }
-    __syncthreads();
-  }
-}
-
 // Sums the planes of the items of a spreading bin that has several (dense
 // bins, up to hundreds of items) into one tile of the bin's planes, so that
 // the reduction below reads one tile per bin.  A workgroup owns one plane of
@@ -773,14 +547,6 @@ template <typename R, int M_>
 void mx_interp3(const cplx<R> *g, cplx<R> *f, const Engine<R> &e, const BinGeom &gg,
                 hipStream_t s, int nb) {
   constexpr int W = 2 * M_ + 2;
-  if constexpr (sizeof(R) == 4) {
-    if (e.mx_dense) {
-      auto fn = e.win.poly_shared ? k_mx_interp3s<W, true> : k_mx_interp3s<W, false>;
-      hipLaunchKernelGGL(fn, dim3((unsigned)e.nsub, (unsigned)nb), dim3(64), 0, s, g, f, e.perm,
-                         e.cell, e.frac, e.subs, gg, e.win);
-      return;
-    }
-  }
   auto fn = e.win.poly_shared ? k_mx_interp3<R, W, true> : k_mx_interp3<R, W, false>;
   hipLaunchKernelGGL(fn, dim3((unsigned)e.nsub, (unsigned)nb), dim3(64 * kMxParts<R>), 0, s, g, f,
                      e.perm, e.cell, e.frac, e.subs, gg, e.win);

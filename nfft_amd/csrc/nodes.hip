@@ -156,20 +156,6 @@ __global__ void k_bins_from_keys(const int *__restrict__ kstart, long nbins, int
   hist[b] = next - first;
 }
 
-// occupied cells: positions where the sorted key changes
-__global__ __launch_bounds__(256) void k_count_cells(const unsigned *__restrict__ key, long M,
-                                                     int *__restrict__ count) {
-  int n = 0;  // (whole wavefronts take every turn)
-  for (long j0 = (long)blockIdx.x * 256; j0 < M; j0 += (long)gridDim.x * 256) {
-    const long j = j0 + threadIdx.x;
-    n += __popcll(__ballot(j < M && (j == 0 || key[j] != key[j - 1])));
-  }
-  __shared__ int sum[4];
-  if ((threadIdx.x & 63) == 0) sum[threadIdx.x >> 6] = n;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(count, sum[0] + sum[1] + sum[2] + sum[3]);
-}
-
 // Planes of every spreading item of a matrix-core plan (items in bin order):
 // from its first node's dimension-0 cell to its last node's, W - 1 more
 __global__ void k_mx_planes(const int4 *__restrict__ items, long nitems,
@@ -631,19 +617,6 @@ void bin_nodes(Engine<R> &e) {
     }
   };
   make_list(e.max_per_sub, 0, sub_start, nsub_of, &e.subs, &e.subs_cap, &e.nsub);
-  // Dense node sets of FP32 matrix-core plans: three nodes or more per
-  // occupied cell, where k_mx_interp3s is the faster B kernel (mx.hpp; the
-  // kooshball holds 5.3)
-  e.mx_dense = false;
-  if (gg.mx && sizeof(R) == 4 && M > 0) {
-    int cells = 0;
-    launch_fill_zero_int(sums + 1, 1, s);
-    hipLaunchKernelGGL(k_count_cells, dim3((unsigned)std::min(2048L, ceil_div(M, 256))), dim3(256), 0, s, key_sorted,
-                       M, sums + 1);
-    NFFT_HIP_CHECK(R, hipMemcpyAsync(&cells, sums + 1, sizeof(int), hipMemcpyDeviceToHost, s));
-    NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
-    e.mx_dense = M >= 3L * cells;
-  }
   // interpolation slots (pairs of same-cell nodes) for the kernels that use them
   e.geom.slots = e.geom.islots = nullptr;
   e.nslots = 0;
