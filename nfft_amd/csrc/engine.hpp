@@ -246,6 +246,12 @@ template <typename R> struct Engine {
   int4 *mx_bin_info = nullptr;
   int *mx_multi = nullptr;
   long mx_bins_cap = 0, mx_multi_n = 0;
+  // matrix-core plans whose B runs on LDS tiles (bin_nodes; mx_b_choice: 0, 1
+  // as the tuner found, -1 by the rule): its bins, slabs of geom's of
+  // interp_geom.bs[0] cells along dimension 0
+  bool mx_tile_b = false;
+  int mx_b_choice = -1;
+  BinGeom interp_geom{};
   // the bins that the LDS-tile kernels would use for a matrix-core plan (d = 0:
   // no such plan), and
   // whether they would run its batches in one launch: the allocation-free

@@ -28,7 +28,8 @@
 //   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.80 + 0.26 (reduction)
 //   B^T, FP64, 2^21 uniform nodes     3.49 + 1.87 ms -> 0.75 + 0.50
 //   B,   FP64, 2^21 uniform nodes     7.03 ms -> 0.96
-//   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.96
+//   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.96; such sets and short
+//     windows keep the LDS tiles, over slabs of these bins (bin_nodes): 1.51
 // FP32 sums are cut so that no product sums more than 128 nodes (B^T) or the 16
 // positions of one plane (B): single sums over an item or a window lost up to a
 // bit (kooshball adjoint 3.0e-7 against FP64, 2.1e-7 as it is and before).

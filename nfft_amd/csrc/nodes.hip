@@ -156,6 +156,20 @@ __global__ void k_bins_from_keys(const int *__restrict__ kstart, long nbins, int
   hist[b] = next - first;
 }
 
+// occupied cells: positions where the sorted key changes
+__global__ __launch_bounds__(256) void k_count_cells(const unsigned *__restrict__ key, long M,
+                                                     int *__restrict__ count) {
+  int n = 0;  // (whole wavefronts take every turn)
+  for (long j0 = (long)blockIdx.x * 256; j0 < M; j0 += (long)gridDim.x * 256) {
+    const long j = j0 + threadIdx.x;
+    n += __popcll(__ballot(j < M && (j == 0 || key[j] != key[j - 1])));
+  }
+  __shared__ int sum[4];
+  if ((threadIdx.x & 63) == 0) sum[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(count, sum[0] + sum[1] + sum[2] + sum[3]);
+}
+
 // Planes of every spreading item of a matrix-core plan (items in bin order):
 // from its first node's dimension-0 cell to its last node's, W - 1 more
 __global__ void k_mx_planes(const int4 *__restrict__ items, long nitems,
@@ -518,7 +532,10 @@ void bin_nodes(Engine<R> &e) {
     ntbins = 1;
     for (int t = 0; t < gg.d; t++) ntbins *= e.tile_geom.nb[t];
   }
-  const long b_bins = al(std::max(nbins, ntbins) * (long)sizeof(int));
+  // B's bins: slabs of the bins where it runs on LDS tiles (the keys of a bin
+  // run over its dimension-0 cells slowest)
+  const long nslabs = gg.mx ? nbins * (gg.bs[0] / e.interp_geom.bs[0]) : nbins;
+  const long b_bins = al(std::max(nslabs, ntbins) * (long)sizeof(int));
   const long b_M = al(M * (long)sizeof(int));
   const long b_cell = al((long)gg.d * M * (long)sizeof(int));
   const long b_frac = al((long)gg.d * M * (long)sizeof(R));
@@ -571,8 +588,6 @@ void bin_nodes(Engine<R> &e) {
                      sums);
   hipLaunchKernelGGL(k_scan_tile_apply, dim3((unsigned)ntiles), dim3(256), 0, s, khist, kstart,
                      nkeys, tile_off);
-  hipLaunchKernelGGL(k_bins_from_keys, dim3((unsigned)ceil_div(nbins, 256)), dim3(256), 0, s,
-                     kstart, nbins, cells_per_bin, (int)M, hist, bin_start);
   if (M > 0) {
     NFFT_HIP_CHECK(R, rocprim::radix_sort_pairs(sort_tmp, sort_bytes, (const unsigned *)key_of,
                                                 key_sorted, rocprim::counting_iterator<int>(0),
@@ -583,15 +598,18 @@ void bin_nodes(Engine<R> &e) {
   // work items of interpolation (small, for balance) and of spreading
   // (larger, to bound the number of tiles written to scratch); the spreading
   // list keeps its per-bin first item and count for the tile reduction
-  auto make_list = [&](int max_per_sub, int max_items, int *first_of, int *count_of, int4 **subs,
-                       long *cap, long *nsub) {
+  int list_totals[2] = {0, 0};  // the list's length and sums[2]
+  auto make_list = [&](long nbins, int max_per_sub, int max_items, int *first_of, int *count_of,
+                       int4 **subs, long *cap, long *nsub) {
+    hipLaunchKernelGGL(k_bins_from_keys, dim3((unsigned)ceil_div(nbins, 256)), dim3(256), 0, s,
+                       kstart, nbins, (int)(nkeys / nbins), (int)M, hist, bin_start);
     hipLaunchKernelGGL(k_count_subs, dim3((unsigned)ceil_div(nbins, 256)), dim3(256), 0, s, hist,
                        nbins, max_per_sub, max_items, count_of);
     hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, count_of, first_of, nbins,
                        sums + 1);
-    int total = 0;
-    NFFT_HIP_CHECK(R, hipMemcpyAsync(&total, sums + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+    NFFT_HIP_CHECK(R, hipMemcpyAsync(list_totals, sums + 1, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
+    const int total = list_totals[0];
     // the list, then the same list in bin order (the ordering's input)
     if (2L * total > *cap) {
       if (*subs) NFFT_HIP_CHECK(R, hipFree(*subs));
@@ -616,11 +634,53 @@ void bin_nodes(Engine<R> &e) {
                          in_bin_order, bucket_of, (long)total, boff, *subs);
     }
   };
-  make_list(e.max_per_sub, 0, sub_start, nsub_of, &e.subs, &e.subs_cap, &e.nsub);
+  // (sums + 2, read back with the list's length: occupied cells)
+  const bool by_cells = gg.mx && gg.m <= 4 && M > 0;
+  if (by_cells) {
+    launch_fill_zero_int(sums + 2, 1, s);
+    hipLaunchKernelGGL(k_count_cells, dim3((unsigned)std::min(2048L, ceil_div(M, 256))), dim3(256), 0,
+                       s, key_sorted, M, sums + 2);
+  }
+  if (nbins > e.bin_arrays_cap) {
+    if (e.sp_first) NFFT_HIP_CHECK(R, hipFree(e.sp_first));
+    NFFT_HIP_CHECK(R, hipMalloc(&e.sp_first, 3 * nbins * sizeof(int)));
+    e.bin_arrays_cap = nbins;
+  }
+  e.sp_count = e.sp_first + nbins;
+  e.bin_order = e.sp_first + 2 * nbins;
+  make_list(nbins, e.spread_max_per_sub, e.spread_max_items, e.sp_first, e.sp_count, &e.sp_subs,
+            &e.sp_subs_cap, &e.sp_nsub);
+  const int cells = list_totals[1];
+  if (gg.mx) {
+    // B on LDS tiles where the nodes per occupied cell reach a limit by window
+    // and precision, for m <= 4: its cost per node grows with W^3, that of the
+    // matrix cores (16 x 16 positions whatever W) little, and its tiles are
+    // loaded whole for few nodes.  Trafo, us, matrix cores / LDS tiles, at 0.03,
+    // 0.3, 1, 3 and 8 uniform nodes per cell (1.02, 1.16, 1.6, 3.2 and 8 per
+    // occupied one), FP32 on 128^3 cells and FP64 on 48 x 64 x 80:
+    //   FP32 m = 2    58 / 64    124 / 85     256 / 115   574 / 251  1436 / 663
+    //   FP32 m = 3    75 / 92    139 / 134    304 / 208   835 / 353  1813 / 877
+    //   FP32 m = 4    95 / 154   152 / 234    328 / 393   792 / 644  2098 / 1380
+    //   FP32 m = 5   132 / 335   205 / 457    428 / 737  1059 / 1369 2763 / 3148
+    //   FP64 m = 2    40 / 46     70 / 52      89 / 66    156 / 93    328 / 145
+    //   FP64 m = 3    43 / 56     74 / 68     112 / 100   205 / 146   465 / 257
+    //   FP64 m = 4    47 / 124    70 / 118    132 / 159   256 / 254   550 / 432
+    constexpr double limit[2][4] = {{1.08, 1.08, 1.12, 2.8}, {1.08, 1.1, 1.3, 4.0}};
+    e.mx_tile_b = e.mx_b_choice == 1;
+    if (e.mx_b_choice < 0 && by_cells)
+      e.mx_tile_b = (double)M >= limit[sizeof(R) == 8][gg.m - 1] * cells;
+    // nodes per item: 2048, on the matrix cores fewer while that leaves less
+    // than 2048 items (they share no tile, and larger ones end the launch late)
+    e.max_per_sub = 2048;
+    while (!e.mx_tile_b && e.max_per_sub > 256 && e.max_per_sub * 2048L > M) e.max_per_sub /= 2;
+  }
+  make_list(gg.mx && e.mx_tile_b ? nslabs : nbins, e.max_per_sub, 0, sub_start, nsub_of, &e.subs,
+            &e.subs_cap, &e.nsub);
   // interpolation slots (pairs of same-cell nodes) for the kernels that use them
-  e.geom.slots = e.geom.islots = nullptr;
+  BinGeom &ig = gg.mx ? e.interp_geom : e.geom;
+  ig.slots = ig.islots = nullptr;
   e.nslots = 0;
-  if (!gg.mx && e.use_slots() && M > 0 && e.nsub > 0) {
+  if ((!gg.mx || e.mx_tile_b) && e.use_slots() && M > 0 && e.nsub > 0) {
     auto long_scan = [&](const int *in, int *out, long len, int *total) {
       const long nt = ceil_div(len, kScanTile);
       hipLaunchKernelGGL(k_scan_tile_sums, dim3((unsigned)nt), dim3(256), 0, s, in, len, tile_sum);
@@ -672,24 +732,15 @@ void bin_nodes(Engine<R> &e) {
     if (e.slot_sort) {
       if (Q == 4)
         hipLaunchKernelGGL(k_sort_slots<4>, dim3((unsigned)e.nsub), dim3(256), 0, s, e.islots,
-                           filled, e.slots, e.cell, M, e.geom.ip2, e.geom.ipp);
+                           filled, e.slots, e.cell, M, ig.ip2, ig.ipp);
       else
         hipLaunchKernelGGL(k_sort_slots<2>, dim3((unsigned)e.nsub), dim3(256), 0, s, e.islots,
-                           filled, e.slots, e.cell, M, e.geom.ip2, e.geom.ipp);
+                           filled, e.slots, e.cell, M, ig.ip2, ig.ipp);
     }
     e.nslots = nslots;
-    e.geom.slots = e.slots;
-    e.geom.islots = e.islots;
+    ig.slots = e.slots;
+    ig.islots = e.islots;
   }
-  if (nbins > e.bin_arrays_cap) {
-    if (e.sp_first) NFFT_HIP_CHECK(R, hipFree(e.sp_first));
-    NFFT_HIP_CHECK(R, hipMalloc(&e.sp_first, 3 * nbins * sizeof(int)));
-    e.bin_arrays_cap = nbins;
-  }
-  e.sp_count = e.sp_first + nbins;
-  e.bin_order = e.sp_first + 2 * nbins;
-  make_list(e.spread_max_per_sub, e.spread_max_items, e.sp_first, e.sp_count, &e.sp_subs,
-            &e.sp_subs_cap, &e.sp_nsub);
   if (gg.mx) {
     // the items' planes and their places in scratch (item counts are at most
     // M, so the node-length temporaries hold them), and what the LDS-tile

@@ -458,12 +458,26 @@ void Engine<R>::set_mx_bins() {
   // nodes per item: up to 2048 (B) and 4096 (B^T, whose two wavefronts share an
   // item and whose tiles are reduced), fewer while that leaves less than 2048
   // items; larger ones end the launch late, smaller ones load and write more
-  // planes (3-D kooshball: B 1.65, 1.55, 1.53 ms with 512, 1024, 2048 nodes;
-  // the reduction 0.73, 0.61, 0.44, 0.37 ms with 512 to 4096)
-  max_per_sub = 2048;
+  // planes (3-D kooshball: the reduction 0.73, 0.61, 0.44, 0.37 ms with 512 to
+  // 4096)
   spread_max_per_sub = 4096;
-  while (max_per_sub > 256 && max_per_sub * 2048L > M) max_per_sub /= 2;
   while (spread_max_per_sub > 512 && spread_max_per_sub * 2048L > M) spread_max_per_sub /= 2;
+  // B on LDS tiles (bin_nodes chooses): slabs of the bins, the thickest whose
+  // tile fits 56 KB; in FP64 48 KB, 64 KB from 8 taps on.  Planes lie 6 cells
+  // further apart than their 16 x 16 cells, which spreads the windows over the
+  // banks.  Trafo, m = 4, 2^24 kooshball nodes: 1.60 ms with slabs of 16 cells,
+  // 1.67 with 8 (2.28 without the 6 cells, 1.80 with rows 20 cells apart); 128^3
+  // cells, FP64, one node per cell, m = 3: 441 us with slabs of 8 cells (63 KB),
+  // 489 with 4; m = 2: 250 (55 KB), 215.
+  BinGeom &ig = interp_geom;
+  ig = geom;
+  ig.ip2 = 16;
+  ig.ipp = 16 * 16 + 6;
+  const int plane = ig.ipp * (int)sizeof(cplx<R>);
+  const int budget = (sizeof(R) == 4 ? 56 : (W >= 8 ? 64 : 48)) * 1024;
+  while (ig.bs[0] % 2 == 0 && (ig.bs[0] + W - 1) * plane > budget) ig.bs[0] /= 2;
+  ig.nb[0] = geom.nb[0] * (geom.bs[0] / ig.bs[0]);
+  ig.E[0] = ig.bs[0] + W - 1;
 }
 
 // Bin edges of 2-D plans on the matrix-core B^T in place of those set by
@@ -1102,9 +1116,22 @@ void Engine<R>::autotune() {
   // bin edges: the default, and the largest edge halved; in 1-D and 2-D also
   // every edge doubled and every edge halved; all within the LDS budget of
   // the default, nodes rebuilt for each, B and B^T timed together
-  // (matrix-core plans have one kernel and one bin shape per window: only
-  // their FFT lines are timed)
+  // (matrix-core plans have one bin shape per window and one B^T: their two B
+  // kernels and the FFT lines are timed)
   const bool tune_b = !geom.mx;
+  if (geom.mx) {
+    const bool dflt = mx_tile_b;
+    float ms[2];
+    for (int c : {dflt ? 0 : 1, dflt ? 1 : 0}) {
+      mx_b_choice = c;
+      build_nodes();
+      ms[c] = time_of([&]() { interp_from_grid(f); });
+    }
+    if (ms[dflt ? 0 : 1] < ms[dflt ? 1 : 0]) {
+      mx_b_choice = dflt ? 0 : 1;
+      build_nodes();
+    }
+  }
   if (tune_b && !std::getenv("NFFT_HIP_BINS") && d <= 3) {
     auto edges = [&]() {
       std::array<int, kMaxDim> e{};
@@ -1244,6 +1271,7 @@ void Engine<R>::autotune() {
     std::fprintf(stderr, " spread=%d item=%d interp=%d fft_shift=%d\n", spread_variant,
                  spread_max_per_sub, interp_variant,
                  fwd_passes.empty() ? 0 : fwd_passes[0].lpb_shift);
+    if (geom.mx) std::fprintf(stderr, "[nfft_hip tune] matrix-core plan, B on %s\n", mx_tile_b ? "LDS tiles" : "matrix cores");
   }
   hipEventDestroy(a);
   hipEventDestroy(b);

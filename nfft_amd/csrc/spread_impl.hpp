@@ -42,6 +42,15 @@ __device__ __forceinline__ int wrap_once(int v, int n) {
 // bin -> lower corner (in cells) of the bin
 template <int D>
 __device__ __forceinline__ void bin_corner(int bin, const BinGeom &gg, int (&lo)[D]) {
+  if constexpr (D == 3) {
+    if (gg.mx) {
+      const int col = bin / gg.nb[0], b1 = col / gg.nb[2];
+      lo[0] = (bin - col * gg.nb[0]) * gg.bs[0];
+      lo[1] = mx_lo(b1, gg.n[1], gg.nb[1]);
+      lo[2] = mx_lo(col - b1 * gg.nb[2], gg.n[2], gg.nb[2]);
+      return;
+    }
+  }
 #pragma unroll
   for (int t = D - 1; t >= 0; t--) {
     lo[t] = (bin % gg.nb[t]) * gg.bs[t];
@@ -1874,11 +1883,15 @@ template <typename R>
 void launch_interp(const cplx<R> *g, cplx<R> *f, const Engine<R> &e, hipStream_t s, int nb,
                    const BinGeom *gb) {
   if (e.nsub == 0) return;
-  if (e.geom.mx) {
+  if (e.geom.mx && !e.mx_tile_b) {
     launch_mx_interp<R>(g, f, e, s, nb, gb);
     return;
   }
-  const BinGeom &gg = gb ? *gb : e.geom;
+  BinGeom gg = e.geom.mx ? e.interp_geom : e.geom;
+  if (gb) {
+    gg.bs_g = gb->bs_g;
+    gg.bs_f = gb->bs_f;
+  }
   size_t lds;
   int threads;
   auto fn = pick_bkernel<R>(bkernels<R>(), gg, false, e.interp_variant, lds, threads,
