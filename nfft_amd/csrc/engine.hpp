@@ -345,8 +345,25 @@ template <typename R> struct Engine {
   // right-hand side needs more than the array holds
   int device = 0;
   void *noalloc_scratch = nullptr;  // device address of the scratch array
-  long noalloc_bytes_per_rhs() const;
-  long noalloc_limit_bytes() const;
+  // bytes of the scratch array that one right-hand side of a batched adjoint
+  // needs: its grid and its spreading tiles, each rounded up to 256 bytes
+  long noalloc_bytes_per_rhs() const {
+    auto up = [](long b) { return (b + 255) / 256 * 256; };
+    return up(n_total * (long)sizeof(cplx<R>)) + up(tile_cells * (long)sizeof(cplx<R>));
+  }
+  // What the entry point's limit is checked against: the bytes of the LDS-tile
+  // kernels' batched adjoint, also for plans with matrix-core bins, so that the
+  // plans it takes do not depend on the kernels (0: no limit, plans those
+  // kernels run one right-hand side at a time).  Where a bound on tile_items
+  // settled the limit: of that bound.
+  long noalloc_limit_bytes() const {
+    if (tile_geom.d == 0) return noalloc_bytes_per_rhs();
+    if (!tile_batchable) return 0;
+    long tot = 1;
+    for (int t = 0; t < d; t++) tot *= tile_geom.E[t];
+    auto up = [](long b) { return (b + 255) / 256 * 256; };
+    return up(n_total * (long)sizeof(cplx<R>)) + up(tile_items * tot * (long)sizeof(cplx<R>));
+  }
   int adjoint_batch_noalloc(const cplx<R> *f_dev, cplx<R> *fhat_dev, int nrhs);
   cplx<R> *bgrid = nullptr;   // batched grids
   cplx<R> *btiles = nullptr;  // batched spreading tiles

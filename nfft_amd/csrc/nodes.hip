@@ -741,6 +741,29 @@ void bin_nodes(Engine<R> &e) {
     ig.slots = e.slots;
     ig.islots = e.islots;
   }
+  // The LDS-tile kernels' items in the bins they would use, for the limit of the
+  // allocation-free batched adjoint: counted where bounds on them (a full item
+  // each 1 / tile_spread_max_per_sub nodes; a bin's last one more) leave open
+  // on which side of it they lie (2^24 kooshball nodes, whose grid alone is
+  // beyond it: 242 us of a precompute)
+  bool count_tiles = false;
+  e.tile_items = 0;
+  if (ntbins > 0 && e.sp_nsub > 0) {
+    auto fits = [&](long items) {
+      e.tile_items = items;
+      return e.noalloc_limit_bytes() <= kNoAllocScratchBytes;
+    };
+    const long most = std::min(M, ntbins + M / e.tile_spread_max_per_sub);
+    const long least = e.spread_max_items > 0 ? 1 : ceil_div(M, e.tile_spread_max_per_sub);
+    count_tiles = !fits(most) && fits(least);
+  }
+  auto launch_count_tiles = [&](int *sum) {
+    launch_fill_zero_int(hist, ntbins, s);
+    hipLaunchKernelGGL(k_tile_bin_hist, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s, e.cell,
+                       e.tile_geom, hist);
+    hipLaunchKernelGGL(k_tile_items, dim3(1), dim3(256), 0, s, hist, ntbins,
+                       e.tile_spread_max_per_sub, e.spread_max_items, sum);
+  };
   if (gg.mx) {
     // the items' planes and their places in scratch (item counts are at most
     // M, so the node-length temporaries hold them), and what the LDS-tile
@@ -771,38 +794,21 @@ void bin_nodes(Engine<R> &e) {
       hipLaunchKernelGGL(k_mx_bin_info, dim3((unsigned)ceil_div(nbins, 256)), dim3(256), 0, s,
                          e.sp_first, e.sp_count, nbins, e.geom, e.mx_info, sums + 1, sums + 2,
                          e.mx_multi, e.mx_bin_info);
-      if (ntbins > 0) {
-        launch_fill_zero_int(hist, ntbins, s);
-        hipLaunchKernelGGL(k_tile_bin_hist, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s,
-                           e.cell, e.tile_geom, hist);
-        hipLaunchKernelGGL(k_tile_items, dim3(1), dim3(256), 0, s, hist, ntbins,
-                           e.tile_spread_max_per_sub, e.spread_max_items, sums + 3);
-      }
+      if (count_tiles) launch_count_tiles(sums + 3);
       NFFT_HIP_CHECK(R, hipMemcpyAsync(totals, sums + 1, 3 * sizeof(int), hipMemcpyDeviceToHost, s));
       NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
     }
     e.mx_multi_n = totals[1];
     e.tile_cells = (totals[0] + (long)totals[1] * (gg.bs[0] + 2 * gg.m + 1)) * 256L;
-    e.tile_items = totals[2];
+    if (count_tiles) e.tile_items = totals[2];
   }
-  if (!gg.mx && ntbins > 0 && e.sp_nsub > 0) {
-    // the LDS-tile kernels' items in the bins they would use: counted where a
-    // bound on them does not settle the limit they serve
-    long tot = 1;
-    for (int t = 0; t < gg.d; t++) tot *= e.tile_geom.E[t];
-    e.tile_items = std::min(M, ntbins + M / e.tile_spread_max_per_sub);
-    if ((tot * e.tile_items + e.n_total) * (long)sizeof(cplx<R>) + 512 > kNoAllocScratchBytes) {
-      int items = 0;
-      launch_fill_zero_int(sums + 1, 1, s);
-      launch_fill_zero_int(hist, ntbins, s);
-      hipLaunchKernelGGL(k_tile_bin_hist, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s, e.cell,
-                         e.tile_geom, hist);
-      hipLaunchKernelGGL(k_tile_items, dim3(1), dim3(256), 0, s, hist, ntbins,
-                         e.tile_spread_max_per_sub, e.spread_max_items, sums + 1);
-      NFFT_HIP_CHECK(R, hipMemcpyAsync(&items, sums + 1, sizeof(int), hipMemcpyDeviceToHost, s));
-      NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
-      e.tile_items = items;
-    }
+  if (!gg.mx && count_tiles) {
+    int items = 0;
+    launch_fill_zero_int(sums + 1, 1, s);
+    launch_count_tiles(sums + 1);
+    NFFT_HIP_CHECK(R, hipMemcpyAsync(&items, sums + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+    NFFT_HIP_CHECK(R, hipStreamSynchronize(s));
+    e.tile_items = items;
   }
   // heavy bins first for the zone reduction (the interpolation list's
   // temporaries are free again: bucket per bin, bucket histogram and offsets)

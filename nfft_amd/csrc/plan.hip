@@ -1034,28 +1034,6 @@ void Engine<R>::adjoint_batch_chunks(const cplx<R> *f_dev, cplx<R> *fhat_dev, in
   NFFT_HIP_CHECK(R, hipGetLastError());
 }
 
-// Bytes of `scratch` that one right-hand side of a batched adjoint needs:
-// its grid and its spreading tiles, each rounded up to 256 bytes.
-template <typename R>
-long Engine<R>::noalloc_bytes_per_rhs() const {
-  auto up = [](long b) { return (b + 255) / 256 * 256; };
-  return up(n_total * (long)sizeof(cplx<R>)) + up(tile_cells * (long)sizeof(cplx<R>));
-}
-
-// What the entry point's limit is checked against: the bytes of the LDS-tile
-// kernels' batched adjoint, also for plans with matrix-core bins, so
-// that the plans it takes do not depend on the kernels (0: no limit, plans
-// those kernels run one right-hand side at a time).
-template <typename R>
-long Engine<R>::noalloc_limit_bytes() const {
-  if (tile_geom.d == 0) return noalloc_bytes_per_rhs();
-  if (!tile_batchable) return 0;
-  long tot = 1;
-  for (int t = 0; t < d; t++) tot *= tile_geom.E[t];
-  auto up = [](long b) { return (b + 255) / 256 * 256; };
-  return up(n_total * (long)sizeof(cplx<R>)) + up(tile_items * tot * (long)sizeof(cplx<R>));
-}
-
 template <typename R>
 int Engine<R>::adjoint_batch_noalloc(const cplx<R> *f_dev, cplx<R> *fhat_dev, int nrhs) {
   const long per = noalloc_bytes_per_rhs();
@@ -1769,7 +1747,7 @@ struct PlanApi {
       }
     }
     if (rc)
-      std::fprintf(stderr, "%sadjoint_batch_device_noalloc: %s (per right-hand side %ld bytes)\n",
+      std::fprintf(stderr, "%sadjoint_batch_device_noalloc: %s (per right-hand side %ld bytes at least)\n",
                    sizeof(R) == 4 ? "nfftf_" : "nfft_", why,
                    e->direct_only ? 0L : e->noalloc_limit_bytes());
     return rc;
