@@ -154,8 +154,8 @@ template <typename R> struct FftPass {
   long gstr[kMaxDim - 1];   // grid strides of the other dimensions
   long fstr[kMaxDim - 1];   // f_hat strides of the other dimensions
   long fstr_ax;   // f_hat stride of dimension t
-  const R *phi_ax;
-  const R *phi_od[kMaxDim - 1];
+  const double *phi_ax;
+  const double *phi_od[kMaxDim - 1];
   long nlines;
   int lines_per_block;  // set by the launch, with twiddle_in_lds
   int nstages;
@@ -214,7 +214,7 @@ template <typename R> struct Engine {
   cplx<R> *fhat = nullptr;
   cplx<R> *f = nullptr;
   R *xdev = nullptr;
-  R *phi_inv = nullptr;  // sum_t N_t scaled deconvolution factors
+  double *phi_inv = nullptr;  // sum_t N_t scaled deconvolution factors
   R *poly = nullptr;     // window polynomials (WinParams::poly)
   int *cell = nullptr;
   R *frac = nullptr;

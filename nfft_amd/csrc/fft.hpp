@@ -396,22 +396,25 @@ __device__ __forceinline__ int band_coord(int k, int n, int N) {
 
 // coordinates of line L0 + ll, the last one fastest: its offsets in the grid
 // and in f_hat and the deconvolution factor of the other dimensions
-template <typename R> struct LineInfo {
+// (the factors are FP64 in both families, a value is multiplied by their
+// rounded product: as FP32 factors, rounded one by one, they made a sixth of
+// the squared error of a 3-D FP32 transform)
+struct LineInfo {
   long in, out;  // offsets in the pass's input and output
-  R fac;
+  double fac;
   int sub;
 };
 
 template <typename R, typename I>
-__device__ __forceinline__ LineInfo<R> line_info(const FftPass<R> &P, I L) {
-  LineInfo<R> li;
+__device__ __forceinline__ LineInfo line_info(const FftPass<R> &P, I L) {
+  LineInfo li;
   li.sub = 0;
   if (P.four) {  // four-step halves: the sub-line index (j1 or k2) runs fastest
     li.sub = (int)(L % (I)P.nsub);
     L /= (I)P.nsub;
   }
   long go = 0, fo = 0;
-  R fac = R(1);
+  double fac = 1.0;
   for (int s = P.nod - 1; s >= 0; s--) {
     const int c = s > 0 ? (int)(L % (I)P.cnt[s]) : (int)L;
     if (s > 0) L /= (I)P.cnt[s];
@@ -485,7 +488,7 @@ __global__ __launch_bounds__(NT, NT > 512 ? 4 : (sizeof(R) == 4 ? 4 : 2)) void k
   extern __shared__ __align__(16) unsigned char fft_smem[];
   cplx<R> *buf = reinterpret_cast<cplx<R> *>(fft_smem);
   cplx<R> *twl = buf + (long)P.lines_per_block * ls;
-  LineInfo<R> *info = reinterpret_cast<LineInfo<R> *>(twl + (P.twiddle_in_lds ? n : 0));
+  LineInfo *info = reinterpret_cast<LineInfo *>(twl + (P.twiddle_in_lds ? n : 0));
   const cplx<R> *tw = P.twiddle;
   if (P.twiddle_in_lds) {
     for (int k = threadIdx.x; k < n; k += blockDim.x) twl[k] = P.twiddle[k];
@@ -508,15 +511,15 @@ __global__ __launch_bounds__(NT, NT > 512 ? 4 : (sizeof(R) == 4 ? 4 : 2)) void k
 
   auto load = [&](int ll, int j, int q, auto &v) {
     constexpr int RAD = sizeof(v) / sizeof(v[0]);
-    const LineInfo<R> &li = info[ll];
+    const LineInfo &li = info[ll];
     const int k0 = ia * j + ib * li.sub;
     if (P.in_mode == kFromCoeffs) {
-      R ph[RAD];
+      double ph[RAD];
 #pragma unroll
       for (int r = 0; r < RAD; r++) {
         const int ks = band_coord(k0 + ia * r * q, nax, P.Nband);
         v[r] = cplx<R>{R(0), R(0)};
-        ph[r] = R(0);
+        ph[r] = 0.0;
         if (ks >= 0) {
           v[r] = fin[li.in + (long)ks * P.fstr_ax];
           ph[r] = P.phi_ax[ks];
@@ -524,7 +527,7 @@ __global__ __launch_bounds__(NT, NT > 512 ? 4 : (sizeof(R) == 4 ? 4 : 2)) void k
       }
 #pragma unroll
       for (int r = 0; r < RAD; r++) {
-        const R f = li.fac * ph[r];
+        const R f = (R)(li.fac * ph[r]);
         v[r] = cplx<R>{v[r].x * f, v[r].y * f};
       }
     } else {
@@ -540,7 +543,7 @@ __global__ __launch_bounds__(NT, NT > 512 ? 4 : (sizeof(R) == 4 ? 4 : 2)) void k
   };
   auto store = [&](int ll, int j, int q, auto &v) {
     constexpr int RAD = sizeof(v) / sizeof(v[0]);
-    const LineInfo<R> &li = info[ll];
+    const LineInfo &li = info[ll];
     const int k0 = oa * j + ob * li.sub;
     if (P.four == 1) {
       // w_n^(j1 k2), stored where its product goes
@@ -562,7 +565,7 @@ __global__ __launch_bounds__(NT, NT > 512 ? 4 : (sizeof(R) == 4 ? 4 : 2)) void k
       for (int r = 0; r < RAD; r++) {
         const int ks = band_coord(k0 + oa * r * q, nax, P.Nband);
         if (ks >= 0) {
-          const R f = li.fac * P.phi_ax[ks];
+          const R f = (R)(li.fac * P.phi_ax[ks]);
           fout[li.out + (long)ks * P.fstr_ax] = cplx<R>{v[r].x * f, v[r].y * f};
         }
       }
@@ -630,7 +633,7 @@ void launch_fft_pass(cplx<R> *g, const cplx<R> *fhat_in, cplx<R> *fhat_out, cons
   }
   const size_t lines = sizeof(cplx<R>) * (size_t)p.lines_per_block * lds_line_stride(p.len);
   const size_t table = sizeof(cplx<R>) * (size_t)p.len;
-  const size_t info = sizeof(LineInfo<R>) * (size_t)p.lines_per_block;
+  const size_t info = sizeof(LineInfo) * (size_t)p.lines_per_block;
   p.twiddle_in_lds = lines + table + info <= (size_t)(big ? 160 : 64) * 1024 ? 1 : 0;
   const size_t lds = lines + info + (p.twiddle_in_lds ? table : 0);
   const long blocks = ceil_div(p.nlines, p.lines_per_block);

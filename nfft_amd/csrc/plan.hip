@@ -149,6 +149,78 @@ static void fit_window_polys(int m, long double b, std::vector<R> &out) {
       out[first + w * (DEG + 1) + i] = (i % 2 ? -1 : 1) * out[first + (2 * m + 1 - w) * (DEG + 1) + i];
 }
 
+// Mean relative change of magnitude by FP32 constants.  An FP32 transform is
+// off by its roundings, which are random, and by a factor: rounded window
+// polynomials and roots of unity make every result some 1e-8 too large or too
+// small per dimension, which adds up over dimensions (150^3 grid, m = 2: 1.4e-7
+// of an error of 2.1e-7).  To first order the factor of a product of steps is
+// the sum of theirs, that of a step with a unitary matrix the mean of
+// conj(exact) (rounded - exact) over its entries; the deconvolution factors are
+// divided by it.
+template <typename R>
+static double window_gain(int m, long double b, const R *poly) {
+  constexpr int DEG = poly_deg_v<R>, K = 8;
+  long double num = 0, den = 0;
+  for (int w = 0; w <= m; w++)  // (the other taps mirror these)
+    for (int j = 0; j < K; j++) {
+      const long double frac = (j + 0.5L) / K, t = frac - 0.5L;
+      const long double exact = psi_scaled(frac + m - w, m, b);
+      long double v = 0;
+      for (int i = DEG; i >= 0; i--) v = v * t + (long double)poly[w * (DEG + 1) + i];
+      num += exact * (v - exact);
+      den += exact * exact;
+    }
+  return (double)(num / den);
+}
+
+// conj(w) (rounded w - w), real part, of the root w = exp(2 pi i k / n)
+template <typename R>
+static double root_gain(long k, long n) {
+  const double a = 2.0 * (double)kPiL * (double)(k % n) / (double)n, c = cos(a), s = sin(a);
+  return c * ((double)(R)c - c) + s * ((double)(R)s - s);
+}
+
+// a butterfly of fft.hpp (dft)
+template <typename R>
+static double butterfly_gain(int rad) {
+  const double h = sqrt(0.5), dh = (double)(R)h / h - 1.0;  // the factor (+-1 +- i) h
+  if (rad == 1 || rad == 2 || rad == 4) return 0.0;
+  if (rad == 8) return 2.0 / 8.0 * dh;
+  static const int split[][3] = {{6, 3, 2}, {9, 3, 3}, {10, 5, 2}, {12, 3, 4}, {15, 5, 3}, {16, 4, 4}};
+  for (const auto &f : split) {
+    if (f[0] != rad) continue;
+    double sum = 0;
+    for (int a = 0; a < f[1]; a++)
+      for (int b = 0; b < f[2]; b++) {
+        const int e = a * b;
+        if (e == 0 || 4 * e == rad) continue;
+        sum += 8 * e == rad || 8 * e == 3 * rad ? dh : root_gain<R>(e, rad);
+      }
+    return butterfly_gain<R>(f[1]) + butterfly_gain<R>(f[2]) + sum / rad;
+  }
+  // a prime: its matrix
+  double sum = 0;
+  for (int k = 1; k < rad; k++)
+    for (int r = 1; r < rad; r++) sum += root_gain<R>((long)r * k, rad);
+  return sum / ((double)rad * rad);
+}
+
+// all stages of a length: butterflies, and the twiddles before each but the first
+template <typename R>
+static double fft_gain(long n, const std::vector<int> &rad) {
+  double g = 0;
+  long Ns = 1;
+  for (int r : rad) {
+    double sum = 0;
+    if (Ns > 1)
+      for (long j = 0; j < Ns; j++)
+        for (int k = 1; k < r; k++) sum += root_gain<R>(j * k, Ns * r);
+    g += butterfly_gain<R>(r) + sum / ((double)Ns * r);
+    Ns *= r;
+  }
+  return g;
+}
+
 // Stages of an FFT of length n (fft.hpp), two at least: for lengths of prime
 // factors up to 13 the fewest radices of 2 .. 13, 15, 16 (each stage more is
 // an LDS pass more), of these the ones with the smallest largest radix and
@@ -547,22 +619,16 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
   NFFT_HIP_CHECK(R, hipMalloc(&frac, sizeof(R) * (size_t)(M > 0 ? M * d : 1)));
   NFFT_HIP_CHECK(R, hipMalloc(&perm, sizeof(int) * (size_t)(M > 0 ? M : 1)));
 
-  // window parameters and scaled deconvolution factors
-  std::vector<R> pinv;
-  for (int t = 0; t < d; t++) {
-    long double sigma = (long double)n[t] / (long double)N[t];
-    long double b = kPiL * (2.0L - 1.0L / sigma);
-    long double peak = sinhl(b * m) / (kPiL * m);  // phi(0)
-    for (long ks = 0; ks < N[t]; ks++) pinv.push_back((R)(peak / phi_hut(n[t], ks - N[t] / 2, m, b)));
-  }
-  NFFT_HIP_CHECK(R, hipMalloc(&phi_inv, sizeof(R) * pinv.size()));
-  NFFT_HIP_CHECK(R, hipMemcpy(phi_inv, pinv.data(), sizeof(R) * pinv.size(), hipMemcpyHostToDevice));
+  // window polynomials
+  double gain[kMaxDim] = {};  // of the window and the FFT, per dimension (FP32)
   {
     std::vector<R> pc;
     for (int t = 0; t < d; t++) {
       long double sigma = (long double)n[t] / (long double)N[t];
       long double b = kPiL * (2.0L - 1.0L / sigma);
+      const size_t at = pc.size();
       fit_window_polys<R>(m, b, pc);
+      if (sizeof(R) == 4) gain[t] = window_gain<R>(m, b, pc.data() + at);
     }
     NFFT_HIP_CHECK(R, hipMalloc(&poly, sizeof(R) * pc.size()));
     NFFT_HIP_CHECK(R, hipMemcpy(poly, pc.data(), sizeof(R) * pc.size(), hipMemcpyHostToDevice));
@@ -669,11 +735,12 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
     NFFT_HIP_CHECK(R, hipMemcpy(dev, tw.data(), sizeof(cplx<R>) * tw.size(), hipMemcpyHostToDevice));
     return dev;
   };
-  auto make_axis = [&](long len) {
+  auto make_axis = [&](long len, int t) {
     FftAxis<R> ax{};
     ax.len = (int)len;
     std::vector<int> rad;
     fft_radices(len, rad);
+    if (sizeof(R) == 4) gain[t] += fft_gain<R>(len, rad);
     ax.nstages = (int)rad.size();
     for (size_t i = 0; i < rad.size(); i++) ax.radix[i] = rad[i];
     std::vector<cplx<R>> tw(len);
@@ -687,7 +754,7 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
   for (int t = 0; t < d; t++) {
     std::vector<int> rad;
     if (n[t] <= cap && fft_radices(n[t], rad)) {
-      axes.push_back(make_axis(n[t]));
+      axes.push_back(make_axis(n[t], t));
       continue;
     }
     // the most balanced n1 n2 = n with both halves fitting and factoring
@@ -705,8 +772,8 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
     split[t] = best;
     axes.push_back(FftAxis<R>{});  // placeholder, the halves carry the tables
     axes.back().len = (int)n[t];
-    sub1[t] = make_axis(n[t] / best);  // first half: length n2
-    sub2[t] = make_axis(best);         // second half: length n1
+    sub1[t] = make_axis(n[t] / best, t);  // first half: length n2
+    sub2[t] = make_axis(best, t);         // second half: length n1
     {
       // w_n^(j1 k2) at k2 n1 + j1, where the first half writes its result
       const long n1 = best, n2 = n[t] / best;
@@ -715,11 +782,28 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
       for (long k2 = 0; k2 < n2; k2++)
         for (long j1 = 0; j1 < n1; j1++) tr[k2 * n1 + j1] = w[j1 * k2];
       tw_full[t] = upload_table(tr);
+      if (sizeof(R) == 4) {
+        double sum = 0;
+        for (const auto &v : tr) sum += sqrt((double)v.x * v.x + (double)v.y * v.y) - 1.0;
+        gain[t] += sum / (double)n[t];
+      }
     }
     extra_twiddles.push_back(sub1[t].twiddle);
     extra_twiddles.push_back(sub2[t].twiddle);
     extra_twiddles.push_back(tw_full[t]);
   }
+  // scaled deconvolution factors, in FP64 for both families: their product over
+  // the dimensions is rounded once
+  std::vector<double> pinv;
+  for (int t = 0; t < d; t++) {
+    long double sigma = (long double)n[t] / (long double)N[t];
+    long double b = kPiL * (2.0L - 1.0L / sigma);
+    long double peak = sinhl(b * m) / (kPiL * m);  // phi(0)
+    for (long ks = 0; ks < N[t]; ks++)
+      pinv.push_back((double)(peak / phi_hut(n[t], ks - N[t] / 2, m, b) / (1.0L + gain[t])));
+  }
+  NFFT_HIP_CHECK(R, hipMalloc(&phi_inv, sizeof(double) * pinv.size()));
+  NFFT_HIP_CHECK(R, hipMemcpy(phi_inv, pinv.data(), sizeof(double) * pinv.size(), hipMemcpyHostToDevice));
   bool four_step = false;
   for (int t = 0; t < d; t++) four_step = four_step || split[t] > 0;
   if (four_step) NFFT_HIP_CHECK(R, hipMalloc(&g2, sizeof(cplx<R>) * (size_t)n_total));
