@@ -80,12 +80,14 @@ constexpr long kNoAllocScratchBytes = 64L << 20;
 
 // 2-D matrix-core B^T (spread_mx2d.hpp): widest tile and window, wavefronts per
 // item, right-hand sides per workgroup of a batch, nodes summed in FP32 before
-// the sums are summed
+// the sums are summed, and the windows for which a wavefront of up to twice as
+// many nodes keeps two sums
 constexpr int kMx2dMaxE = 48;
 constexpr int kMx2dMaxM = 8;
 template <typename R> constexpr int kMx2dWaves = sizeof(R) == 4 ? 4 : 2;
 constexpr int kMx2dRhs = 2;
-constexpr int kMx2dOneSum = 64;
+constexpr bool mx2d_two_sums(int m) { return m <= 3 || m >= 6; }
+constexpr int kMx2dOneSum = 32;
 
 // Kaiser-Bessel window of one dimension, scaled by 1/phi(0) so that the B
 // weights stay O(1) (the scale is folded into the deconvolution factors).

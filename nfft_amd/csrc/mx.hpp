@@ -75,9 +75,11 @@ __global__ __launch_bounds__(128, sizeof(R) == 4 ? (W <= 10 ? 4 : 3) : 2) void k
     mx_load_poly<R, 3, W>(spoly, wp.poly, threadIdx.x, 128);
     __syncthreads();
   }
-  // FP32: a product's sum runs over 4 chunks, the sums of these over the item
-  // (one sum over the thousands of nodes of a dense item would lose a bit)
+  // FP32: a product's sum runs over 4 chunks (2 where more nodes reach a cell),
+  // the sums of these over the item (one sum over the thousands of nodes of a
+  // dense item would lose a bit)
   constexpr bool TWO = sizeof(R) == 4;
+  constexpr int FOLD = W >= 14 ? 2 : 4;
   mx4<R> acc[H][2], sum[TWO ? H : 1][2];
 #pragma unroll
   for (int i = 0; i < H; i++) {
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(128, sizeof(R) == 4 ? (W <= 10 ? 4 : 3) : 2) void k
       k = end;
     }
     if constexpr (TWO) {
-      if ((base / NC) % 4 == 3) {
+      if ((base / NC) % FOLD == FOLD - 1) {
 #pragma unroll
         for (int s = 0; s < H; s++)
 #pragma unroll
@@ -408,11 +410,13 @@ __global__ __launch_bounds__(256) void k_mx_sum3(cplx<R> *__restrict__ tiles,
 #pragma unroll
       for (int u = 0; u < 8; u++)
         v[u] = i + u < n ? tiles[(long)list[i + u] * 256 + threadIdx.x] : cplx<R>{0, 0};
+      // (in pairs first: shorter FP32 sums)
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        ar += v[u].x;
-        ai += v[u].y;
-      }
+      for (int w = 1; w < 8; w *= 2)
+#pragma unroll
+        for (int u = 0; u < 8; u += 2 * w) v[u] = cplx<R>{v[u].x + v[u + w].x, v[u].y + v[u + w].y};
+      ar += v[0].x;
+      ai += v[0].y;
     }
     __syncthreads();
   }

@@ -1616,13 +1616,21 @@ __global__ __launch_bounds__(256) void k_gather_zones_cell(const cplx<R> *__rest
           v[u][z] = cplx<R>{0, 0};
           if (c + u < cnt[z]) v[u][z] = tp[z][rt + (long)(c + u) * tot];
         }
+      // summed in pairs first: as one chain over hundreds of values the FP32 sum
+      // was the largest error of dense sets
 #pragma unroll
-      for (int u = 0; u < U; u++)
+      for (int w = 1; w < U; w *= 2)
 #pragma unroll
-        for (int z = 0; z < NZ; z++) {
-          ar += v[u][z].x;
-          ai += v[u][z].y;
-        }
+        for (int u = 0; u + w < U; u += 2 * w)
+#pragma unroll
+          for (int z = 0; z < NZ; z++) v[u][z] = cplx<R>{v[u][z].x + v[u + w][z].x, v[u][z].y + v[u + w][z].y};
+#pragma unroll
+      for (int w = 1; w < NZ; w *= 2)
+#pragma unroll
+        for (int z = 0; z + w < NZ; z += 2 * w)
+          v[0][z] = cplx<R>{v[0][z].x + v[0][z + w].x, v[0][z].y + v[0][z + w].y};
+      ar += v[0][0].x;
+      ai += v[0][0].y;
     }
     if (q < core) gp[(long)r * gg.bs_g] = cplx<R>{ar, ai};
   }
@@ -1702,7 +1710,8 @@ template <typename R> struct BKernelTable {
   fn spread_runs2d_mc[kMaxStaticM + 1];       // same, kRhsPerGroup right-hand sides each
   // d = 2 on the matrix cores: [blocks per dimension - 2][window table shared]
   // [sums of sums, float]; two blocks of single sums with kMx2dRhs right-hand
-  // sides per workgroup (float; the others would take over half the registers)
+  // sides per workgroup (float, m = 4, 5; the others would take over half the
+  // registers)
   fn spread_mx2d[2][2][2][kMx2dMaxM + 1];
   fn spread_mx2d_mc[2][kMx2dMaxM + 1];
   fn interp_rt[kMaxDim][2];  // [d-1][tile]
@@ -1735,7 +1744,7 @@ void bk_fill_one(BKernelTable<R> &k) {
     k.spread_mx2d[0][1][1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, 1, true, TWO>;
     k.spread_mx2d[1][0][1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 3, 1, false, TWO>;
     k.spread_mx2d[1][1][1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 3, 1, true, TWO>;
-    if constexpr (std::is_same_v<R, float>) {
+    if constexpr (std::is_same_v<R, float> && !mx2d_two_sums(M_)) {
       k.spread_mx2d_mc[0][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, kMx2dRhs, false, false>;
       k.spread_mx2d_mc[1][M_] = k_spread_mx2d<R, 2 * M_ + 2, 2, kMx2dRhs, true, false>;
     }
@@ -1912,14 +1921,14 @@ void launch_spread(const cplx<R> *f, cplx<R> *g, const Engine<R> &e, hipStream_t
   size_t lds;
   int threads;
   const bool shared_poly = e.win.poly_shared != 0;
-  // items of more nodes than kMx2dOneSum per wavefront
-  const bool two_sums = e.spread_max_per_sub > kMx2dOneSum * kMx2dWaves<R> || e.spread_max_items > 0;
+  // items of more nodes than two kMx2dOneSum per wavefront
+  const bool two_sums = e.spread_max_per_sub > 2 * kMx2dOneSum * kMx2dWaves<R> || e.spread_max_items > 0;
   auto fn = pick_bkernel<R>(bkernels<R>(), gg, true, e.spread_variant, lds, threads, shared_poly,
                             two_sums);
   const int blocks = mx2d_blocks(gg, e.spread_variant);
   // the scratch reduction needs a tile per item; the global variant adds directly
   if (!tiles) tiles = ((lds > 0 || blocks) && e.tile_scratch) ? e.tiles : nullptr;
-  if (nb > 1 && blocks == 2 && !two_sums) {
+  if (nb > 1 && blocks == 2 && !two_sums && !mx2d_two_sums(gg.m)) {
     // as below, kMx2dRhs right-hand sides per workgroup
     BinGeom gm = gg;
     gm.nrhs = nb;

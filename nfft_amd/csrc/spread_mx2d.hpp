@@ -23,9 +23,14 @@
 // Measured per launch, against the run-merging kernel (FP32) and LDS atomics
 // (FP64): 2^20 clustered nodes on 1024^2, m = 4 FP32 138 -> 62 us, m = 6 FP64
 // 577 -> 154; 128512 radial nodes on 512^2, m = 4 FP32 30 -> 14; 32 right-hand
-// sides of 206336 such nodes 441 -> 306.  Errors against FP64 are those of the
-// kernels before (m = 4, 600 x 500: 1.75e-7 and 1.79e-7), with sums over at most
-// kMx2dOneSum nodes; over 128 and 256 nodes they grew by a tenth and a fifth.
+// sides of 206336 such nodes 441 -> 306.
+//
+// FP32 errors against FP64, adjoint on 256^2 cells with 2^18 radial nodes (1e-7;
+// kernels before / one sum over 64 nodes / two): m = 2 1.32 / 1.36 / 1.29, m = 3
+// 1.38 / 1.41 / 1.34, m = 4 1.54 / 1.56, m = 5 1.94 / 1.83, m = 6 2.07 / 2.21 /
+// 2.07.  Two sums cost single right-hand sides nothing and batches their second
+// right-hand side per workgroup (registers): 32 of 206336 nodes, m = 3, 359 ->
+// 429 us (467 with both).
 #pragma once
 
 #include "mx_util.hpp"
@@ -69,10 +74,13 @@ __global__ __launch_bounds__(64 * kMx2dWaves<R>, sizeof(R) == 8 && T == 3 && !SH
   // the wavefront's share of the nodes, whole groups of four
   const int part = ((sp.z + NWV - 1) / NWV + 3) & ~3;
   const int first = min(sp.z, wv * part), cntw = min(sp.z, first + part) - first;
-  // TWO (FP32, long shares): a product's sum runs over kMx2dOneSum nodes, the
-  // sums of these over the share (one sum over all nodes of a dense cell would
-  // lose up to a bit)
-  mx4<R> acc[NR][T][T][2], sum[TWO ? NR : 1][TWO ? T : 1][TWO ? T : 1][2];
+  // FP32 sums over at most kMx2dOneSum nodes (one sum over all nodes of a dense
+  // cell would lose up to a bit).  TWO, long shares: the sums of these run over
+  // the share.  Shares of up to twice as many: groups of four add to two sums
+  // in turn, except where one is no further off than the kernels before (see
+  // the head) or registers lack (three blocks).
+  constexpr int H = sizeof(R) == 4 && !TWO && T == 2 && mx2d_two_sums(W / 2 - 1) ? 2 : 1;
+  mx4<R> acc[H][NR][T][T][2], sum[TWO ? NR : 1][TWO ? T : 1][TWO ? T : 1][2];
 #pragma unroll
   for (int c = 0; c < NR; c++)
 #pragma unroll
@@ -81,7 +89,8 @@ __global__ __launch_bounds__(64 * kMx2dWaves<R>, sizeof(R) == 8 && T == 3 && !SH
       for (int b = 0; b < T; b++)
 #pragma unroll
         for (int x = 0; x < 2; x++) {
-          acc[c][a][b][x] = mx4<R>{0, 0, 0, 0};
+#pragma unroll
+          for (int h = 0; h < H; h++) acc[h][c][a][b][x] = mx4<R>{0, 0, 0, 0};
           if constexpr (TWO) sum[c][a][b][x] = mx4<R>{0, 0, 0, 0};
         }
   auto fold = [&]() {
@@ -96,8 +105,8 @@ __global__ __launch_bounds__(64 * kMx2dWaves<R>, sizeof(R) == 8 && T == 3 && !SH
             for (int x = 0; x < 2; x++)
 #pragma unroll
               for (int i = 0; i < 4; i++) {
-                sum[c][a][b][x][i] += acc[c][a][b][x][i];
-                mx_clear(acc[c][a][b][x], i);
+                sum[c][a][b][x][i] += acc[0][c][a][b][x][i];
+                mx_clear(acc[0][c][a][b][x], i);
               }
     }
   };
@@ -148,7 +157,8 @@ __global__ __launch_bounds__(64 * kMx2dWaves<R>, sizeof(R) == 8 && T == 3 && !SH
         pnext = permp[min(base + 2 * NC + me, last)];
       }
       __builtin_amdgcn_wave_barrier();
-      for (int k = 0; k < cnt; k += 4) {
+      auto four = [&](int k, auto set) {
+        constexpr int h = decltype(set)::value;
         const R *row = win + (k + q) * P + j;
         R p0[T], p1[T];
 #pragma unroll
@@ -173,11 +183,16 @@ __global__ __launch_bounds__(64 * kMx2dWaves<R>, sizeof(R) == 8 && T == 3 && !SH
             if (((reach[a] >> k) & 15) == 0) continue;
 #pragma unroll
             for (int r = 0; r < NR; r++) {
-              acc[r][a][b][0] = mx_mul(p0[a], br[r], acc[r][a][b][0]);
-              acc[r][a][b][1] = mx_mul(p0[a], bi[r], acc[r][a][b][1]);
+              acc[h][r][a][b][0] = mx_mul(p0[a], br[r], acc[h][r][a][b][0]);
+              acc[h][r][a][b][1] = mx_mul(p0[a], bi[r], acc[h][r][a][b][1]);
             }
           }
         }
+      };
+      for (int k = 0; k < cnt; k += 4 * H) {
+        four(k, std::integral_constant<int, 0>{});
+        if constexpr (H == 2)
+          if (k + 4 < cnt) four(k + 4, std::integral_constant<int, 1>{});
       }
       __builtin_amdgcn_wave_barrier();
       if ((base + NC) % kMx2dOneSum == 0 && base + NC < cntw) fold();
@@ -199,7 +214,8 @@ __global__ __launch_bounds__(64 * kMx2dWaves<R>, sizeof(R) == 8 && T == 3 && !SH
           for (int i = 0; i < 4; i++) {
             const int e0 = 16 * a + mx_row<R>(q, i), e1 = 16 * b + j;
             if (e0 < E0 && e1 < E1) {
-              C s = C{acc[r][a][b][0][i], acc[r][a][b][1][i]};
+              C s = C{acc[0][r][a][b][0][i], acc[0][r][a][b][1][i]};
+              if constexpr (H == 2) s = C{s.x + acc[1][r][a][b][0][i], s.y + acc[1][r][a][b][1][i]};
               if constexpr (TWO) s = C{s.x + sum[r][a][b][0][i], s.y + sum[r][a][b][1][i]};
               if (w > 0) {
                 const C o = tile[e0 * E1 + e1];
