@@ -564,6 +564,16 @@ template <typename R>
 void Engine<R>::set_mx2d_bins() {
   if (d != 2 || spread_variant != 15 || m < 1 || m > kMx2dMaxM) return;
   const int W = 2 * m + 2;
+  // Windows of three blocks (bins of 16 cells, tiles of 33): few nodes on large
+  // zoned bins keep those and their kernels, whose tiles are 2.3 times the
+  // grid instead of 4.3 (m = 8, adjoint, these / 16 cells: 4096^2 FP32 with 0.05
+  // nodes per cell 0.85 / 1.84 ms, FP64 1.63 / 2.53; 1024^2 FP32 with 0.1 86 /
+  // 123 us, with 1 461 / 189; with 0.13 4096^2 FP32 1.32 / 1.93 ms, 1024^2 FP64,
+  // both directions, 221 / 247 us)
+  if (W > 16 && geom.zoned && std::max(geom.bs[0], geom.bs[1]) > 16 && M * 6 < n_total) {
+    spread_variant = sizeof(R) == 4 ? 14 : 1;
+    return;
+  }
   int bs[kMaxDim];
   for (int t = 0; t < kMaxDim; t++) bs[t] = 1;
   for (int t = 0; t < d; t++) {
@@ -710,8 +720,9 @@ void Engine<R>::create(int d_, const long *N_, const long *n_, long M_, int m_) 
   // 2-D: matrix cores (tiles wider than kMx2dMaxE cells and windows beyond
   // kMx2dMaxM: as follows).  float: plain FP32 read-modify-write by wavefronts
   // that own disjoint cells, same-cell runs summed in registers (3-D: two
-  // wavefronts per tile split by row parity; 2-D: one wavefront per tile; 1-D:
-  // private tiles); double: wavefronts sharing a tile with ds_add_f64
+  // wavefronts per tile split by row parity; 2-D: two wavefronts with a tile
+  // each, added up when it is written; 1-D: private tiles); double: wavefronts
+  // sharing a tile with ds_add_f64
   spread_variant = variant("NFFT_HIP_SPREAD", d == 2 ? 15 : (sizeof(R) == 4 ? (d == 3 ? 10 : 2) : 1));
 
   set_mx_bins();
