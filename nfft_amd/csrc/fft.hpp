@@ -623,7 +623,7 @@ void launch_fft_pass(cplx<R> *g, const cplx<R> *fhat_in, cplx<R> *fhat_out, cons
   const long fit_big = std::min<long>(256, 4 * fft_cap<R>() / p.len);
   const bool big = strided && !generic && fft_cap<R>() / p.len < seg && p.nlines * (long)nb / fit_big >= 256;
   if (big) {
-    p.lines_per_block = (int)fit_big;
+    p.lines_per_block = (int)std::max(std::min(4L, fit_big), fit_big >> std::max(0, -p0.lpb_shift));
   } else {
     const long fit = std::max<long>(1, std::min<long>(256, fft_cap<R>() / p.len));
     long want = std::max<long>(1, p0.nlines * (long)nb / 1024);
