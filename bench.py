@@ -574,7 +574,7 @@ def main():
     if b_adj_ms >= b_trafo_ms:
         dom_name, dom_ms, dom_sym = "B^T spreading (k_mx_spread3, adjoint)", b_adj_ms, "k_mx_spread3"
     else:
-        dom_name, dom_ms, dom_sym = "B interpolation (k_mx_interp3s, trafo)", b_trafo_ms, "k_mx_interp3s"
+        dom_name, dom_ms, dom_sym = "B interpolation (k_interp_tile, trafo)", b_trafo_ms, "k_interp_tile"
     # HBM bytes per launch of that kernel measured by rocprofv3 FETCH_SIZE /
     # WRITE_SIZE (copy-calibrated) and committed with the profile summaries
     # (the profile names the exact kernel each stage ran in its run)
@@ -600,6 +600,18 @@ def main():
         tf = 4.0 * taps / (ms * 1e-3) / 1e12
         return {"taps": taps, "lds_GBs": lds, "lds_frac": lds / LDS_PEAK_GBS,
                 "fma_TFLOPs": tf, "valu_frac": tf / VALU_FP32_TFLOPS}
+
+    # What bounds the longest stage.  B^T: the FP32 matrix products it issues,
+    # (2m+2) planes x 2 parts of 16 x 16 multiply-adds per node, of which
+    # ((2m+2)/16)^2 meet a nonzero window (they run at the FP32 vector peak's
+    # rate).  B: the taps' multiply-adds on the vector ALUs.
+    if dom_sym == "k_mx_spread3":
+        flops, roof_peak, roof_bound = 2.0 * (2 * m + 2) * 2 * 256 * M, FP32_PEAK_TFLOPS, "mfma"
+    else:
+        flops, roof_peak, roof_bound = 4.0 * taps, VALU_FP32_TFLOPS, "valu"
+    tf = flops / (dom_ms * 1e-3) / 1e12
+    roof = {"bound": roof_bound, "achieved": tf, "peak": roof_peak, "unit": "TFLOP/s",
+            "frac": tf / roof_peak, "flops_issued_per_launch": flops}
 
     stages = {
         "trafo_D_FFT": hbm(ab["D"] + ab["F"], stages_ms["trafo_D"] + stages_ms["trafo_FFT"]),
@@ -636,37 +648,27 @@ def main():
             "N": N, "n": n, "m": m, "M": M, "parallelism": "single GPU",
             "planning": "FFTW_ESTIMATE" if args.estimate else "FFTW_MEASURE",
         },
-        "roofline": {
-            "bound": "hbm",
-            "kernel": dom_name,
-            "achieved": achieved,
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS,
-            "traffic": traffic,
-            "traffic_source": "profiles/traffic_kooshball3d.json (rocprofv3 FETCH_SIZE + WRITE_SIZE "
-                              "per dispatch, scaled by a 1 GiB copy kernel's readings)",
-            "avg_launch_ms": dom_ms,
-            "algorithmic_bytes_per_launch": ab["B"],
-            # the same launch against the on-chip peak that bounds it: 4
-            # flops per tap (complex value times real weight), (2m+2)^d taps
-            # per node, against the published FP32 vector peak (157.3 TFLOP/s,
-            # which counts packed FP32) and the unpacked FMA issue rate this
-            # library's code runs at (78.6 TFLOP/s)
-            "onchip": {
-                "bound": "valu",
-                "achieved": 4.0 * taps / (dom_ms * 1e-3) / 1e12,
-                "peak": FP32_PEAK_TFLOPS,
-                "unit": "TFLOP/s",
-                "frac": 4.0 * taps / (dom_ms * 1e-3) / 1e12 / FP32_PEAK_TFLOPS,
-                "frac_of_unpacked_fma": 4.0 * taps / (dom_ms * 1e-3) / 1e12 / VALU_FP32_TFLOPS,
-                "flops_per_launch": 4.0 * taps,
-            },
-            # which of the two fractions is higher, i.e. the roof this kernel
-            # is nearer to
-            "limiter": ("valu" if 4.0 * taps / (dom_ms * 1e-3) / 1e12 / FP32_PEAK_TFLOPS
-                        > achieved / HBM_PEAK_GBS else "hbm"),
-        },
+        "roofline": dict(
+            roof,
+            kernel=dom_name,
+            traffic=traffic,
+            traffic_source="profiles/traffic_kooshball3d.json (rocprofv3 FETCH_SIZE + WRITE_SIZE "
+                           "per dispatch, scaled by a 1 GiB copy kernel's readings)",
+            avg_launch_ms=dom_ms,
+            algorithmic_bytes_per_launch=ab["B"],
+            hbm={"achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                 "frac": achieved / HBM_PEAK_GBS},
+            # the taps alone: 4 flops per tap (complex value times real
+            # weight), (2m+2)^d taps per node, against the published FP32
+            # vector peak (157.3 TFLOP/s, which counts packed FP32) and the
+            # unpacked FMA issue rate this library's code runs at (78.6)
+            taps={"achieved": 4.0 * taps / (dom_ms * 1e-3) / 1e12,
+                  "peak": FP32_PEAK_TFLOPS,
+                  "unit": "TFLOP/s",
+                  "frac": 4.0 * taps / (dom_ms * 1e-3) / 1e12 / FP32_PEAK_TFLOPS,
+                  "frac_of_unpacked_fma": 4.0 * taps / (dom_ms * 1e-3) / 1e12 / VALU_FP32_TFLOPS,
+                  "flops_per_launch": 4.0 * taps},
+        ),
         "step_hbm": {
             "algorithmic_bytes": step_bytes,
             "achieved_GBs": step_bytes / (ms_step * 1e-3) / 1e9,

@@ -25,14 +25,14 @@
 // 5.5 cycles each between FP32 products), so the kernels are built to issue
 // few of them per node.  Measured against the LDS-tile kernels (spread_impl.hpp,
 // spread_runs.hpp), m = 4, 256^3 grid:
-//   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.80 + 0.26 (reduction)
+//   B^T, FP32, 2^24 kooshball nodes   4.01 + 0.25 ms -> 1.77 + 0.27 (reduction)
 //   B^T, FP64, 2^21 uniform nodes     3.49 + 1.87 ms -> 0.75 + 0.50
 //   B,   FP64, 2^21 uniform nodes     7.03 ms -> 0.96
 //   B,   FP32, 2^24 kooshball nodes   1.62 ms -> 1.96; such sets and short
-//     windows keep the LDS tiles, over slabs of these bins (bin_nodes): 1.51
+//     windows keep the LDS tiles, over slabs of these bins (bin_nodes): 1.53
 // FP32 sums are cut so that no product sums more than 128 nodes (B^T) or the 16
 // positions of one plane (B): single sums over an item or a window lost up to a
-// bit (kooshball adjoint 3.0e-7 against FP64, 2.1e-7 as it is and before).
+// bit (kooshball adjoint 3.0e-7 against FP64, 1.9e-7 as it is).
 // FP64 on sparse nodes (6 per column and plane) is bound by its grid traffic:
 // 256 / 49 grid cells read or written per cell, 41 planes per 32.
 #pragma once
